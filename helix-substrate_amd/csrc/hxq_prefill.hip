@@ -48,8 +48,53 @@
 #include <type_traits>
 
 #include "hxq_common.h"
+#include "hxq_rows.h"
 
 namespace hxq {
+namespace rw {
+
+// The few-row plan of a call (mt 0: the tiled kernel runs).
+//
+// Where the line lies: up to 128 rows (two blocks of 64 per run of W) always,
+// above that while the 16-row subtiles of W times the 64-row blocks of X stay
+// within three per CU, two where K is above 8192 (X is read again by every
+// block).  Measured, us, tiled against few-row: 16 x 18944 x 3584 (M, OUT, K)
+// 60.1 / 24.2, 16 x 3584 x 18944 70.0 / 29.6, 64 x 18944 x 3584 61.5 / 33.8,
+// 64 x 3584 x 18944 71.1 / 50.5, 128 x 8512 x 2048 40.2 / 23.0, 512 x 512 x
+// 3584 23.1 / 14.4, 192 x 3584 x 3584 28.0 / 24.4; past the line 256 x 3584 x
+// 3584 28.9 / 32.4, 512 x 2048 x 4096 32.3 / 35.2.  fp32 X (32-row blocks):
+// 16 x 18944 x 3584 174 / 38.6, 64 x 3584 x 3584 69.5 / 26.7.
+//
+// Subtiles per block: one block runs per CU, so a block count is rounds of the
+// chip, and each round costs a fixed part (table, first loads, final sum: the
+// time of about 6000 columns of one subtile) besides its subtiles.
+Plan plan(int64_t m, int64_t out, int64_t in, bool f32, bool affine, int32_t group, int format, int cus) {
+    Plan p{};
+    if (affine && group >= 16384 && group < in) return p;  // group index by one multiply
+    const int64_t most = f32 ? kMaxRowsF32 : kMaxRows;
+    const int64_t by = (m + most - 1) / most;
+    const int64_t subs = (out + kSub - 1) / kSub;
+    if (by > 2 && subs * by > (in > 8192 ? 2 : 3) * cus) return p;
+    const int64_t rows = (m + by - 1) / by;
+    p.by = static_cast<int>(by);
+    p.mt = static_cast<int>((rows + kSub - 1) / kSub);
+    double cost = 0;
+    for (int ns : {1, 2, 3, 5}) {
+        if (ns > 3 && format == HXQ_FMT_SCALAR_U16) break;  // two index loads: registers
+        const int64_t blocks = (subs + ns - 1) / ns * by;
+        const double c = static_cast<double>((blocks + cus - 1) / cus) * (ns * static_cast<double>(in) + 6000.0);
+        if (ns == 1 || c < cost) {
+            cost = c;
+            p.ns = ns;
+        }
+    }
+    p.bx = static_cast<int>((subs + p.ns - 1) / p.ns);
+    p.sp = p.ns == 1 ? (p.mt == 1 && in > 4096 ? 4 : 2) : p.ns == 2 && p.mt == 1 ? 2 : 1;
+    return p;
+}
+
+}  // namespace rw
+
 namespace pg {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -1008,6 +1053,7 @@ extern "C" int64_t hxq_prefill_gemm_workspace_bytes(int64_t m_rows, int64_t out_
                                                     int64_t in_features) {
     if (m_rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % pg::kBK) return 0;
     // the largest over the row-tile heights a format may use
+    if (m_rows <= rw::kMaxRows && in_features < 16384) return 0;  // the few-row kernel, every format and type
     const int cus = device_cu_count();
     return std::max(pg::plan(m_rows, out_features, in_features, cus).ws_bytes,
                     pg::plan(m_rows, out_features, in_features, cus, 128).ws_bytes);
@@ -1050,6 +1096,33 @@ extern "C" int hxq_prefill_gemm(const void *x, int32_t x_dtype, int32_t format,
     HXQ_REQUIRE((reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
                     (reinterpret_cast<uintptr_t>(indices) & 15u) == 0,
                 "x and indices must be 16-byte aligned");
+    const rw::Plan rp = rw::plan(m_rows, out_features, in_features, x_dtype == HXQ_F32, group_affine != nullptr,
+                                 group_size, format, device_cu_count());
+    if (rp.mt > 0) {
+        rw::Call r{};
+        r.x = x;
+        r.idx = indices;
+        r.cb = codebook;
+        r.ga = reinterpret_cast<const float2 *>(group_affine);
+        r.a.sc_ptr = sc_grp_ptr;
+        r.a.sc_key = sc_grp_key;
+        r.a.sc_val = sc_grp_val;
+        r.a.bias = bias;
+        r.a.y = y;
+        r.M = static_cast<int32_t>(m_rows);
+        r.OUT = static_cast<int32_t>(out_features);
+        r.K = static_cast<int32_t>(in_features);
+        r.a.n_codes = n_codes;
+        r.a.y_dtype = y_dtype;
+        r.ngroups = static_cast<int32_t>(ngroups);
+        const uint32_t gd = group_affine ? static_cast<uint32_t>(group_size / 16) : 1u;
+        r.gmul = gd == 1 ? 0u : group_size >= in_features ? 1u : static_cast<uint32_t>(((uint64_t{1} << 32) + gd - 1) / gd);
+        r.a.vec_out = out_features % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+        const bool aff = group_affine != nullptr;
+        if (x_dtype == HXQ_BF16) return rw::launch_rows<1>(r, format, aff, rp, stream);
+        if (x_dtype == HXQ_F16) return rw::launch_rows<0>(r, format, aff, rp, stream);
+        return rw::launch_rows<2>(r, format, aff, rp, stream);
+    }
     // uint16 scalar indices with the affine need more registers than the
     // 256-row tile leaves: 128-row tiles
     // fp32 activations: 128-row tiles (the fp32 A tile doubles the LDS)

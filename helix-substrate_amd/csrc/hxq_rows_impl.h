@@ -1,0 +1,63 @@
+// Instantiations of the few-row GEMM for one activation type (included by
+// hxq_rows_bf16.hip, hxq_rows_f16.hip and hxq_rows_f32.hip, which build in parallel).
+#pragma once
+#include <type_traits>
+
+#include "hxq_rows.h"
+
+namespace hxq {
+namespace rw {
+
+template <int XT, int MT, int NS, int SP, int W>
+static int launch_fmt(const Call &c, int format, bool aff, const Plan &p, hipStream_t stream) {
+    const dim3 grid(p.bx, p.by), block(W * 64);
+#define HXQ_RW(AF_, F_) \
+    hipLaunchKernelGGL((rows_kernel<MT, NS, SP, XT, AF_, F_, W>), grid, block, 0, stream, c.idx, c.x, c.cb, \
+                       c.ga, c.M, c.OUT, c.K, c.ngroups, c.gmul, c.a)
+    switch (format) {
+        case HXQ_FMT_SCALAR:
+            if (aff) HXQ_RW(true, HXQ_FMT_SCALAR); else HXQ_RW(false, HXQ_FMT_SCALAR);
+            break;
+        case HXQ_FMT_SCALAR_U16:
+            if (aff) HXQ_RW(true, HXQ_FMT_SCALAR_U16); else HXQ_RW(false, HXQ_FMT_SCALAR_U16);
+            break;
+        case HXQ_FMT_VQ2_U16: HXQ_RW(false, HXQ_FMT_VQ2_U16); break;
+        case HXQ_FMT_VQ2_P12: HXQ_RW(false, HXQ_FMT_VQ2_P12); break;
+        default: HXQ_RW(true, HXQ_FMT_AF6); break;
+    }
+#undef HXQ_RW
+    HXQ_LAUNCH_CHECK();
+    return HXQ_OK;
+}
+
+// fp32 X takes twice the registers: eight waves, so that 256 are there for each
+template <int XT>
+int launch_rows(const Call &c, int format, bool aff, const Plan &p, hipStream_t stream) {
+    constexpr int W = XT == 2 ? 8 : 16;
+#define HXQ_RWS(MT_, NS_, SP_, W_) \
+    if (p.mt == MT_ && p.ns == NS_ && p.sp == SP_) return launch_fmt<XT, MT_, NS_, SP_, W_>(c, format, aff, p, stream)
+    HXQ_RWS(1, 1, 2, W);
+    HXQ_RWS(1, 1, 4, W);
+    HXQ_RWS(1, 2, 2, W);
+    HXQ_RWS(1, 3, 1, W);
+    HXQ_RWS(1, 5, 1, W);
+    HXQ_RWS(2, 1, 2, W);
+    HXQ_RWS(2, 2, 1, W);
+    HXQ_RWS(2, 3, 1, W);
+    HXQ_RWS(2, 5, 1, 8);
+    if constexpr (XT != 2) {
+        HXQ_RWS(3, 1, 2, 8);
+        HXQ_RWS(3, 2, 1, 8);
+        HXQ_RWS(3, 3, 1, 8);
+        HXQ_RWS(3, 5, 1, 8);
+        HXQ_RWS(4, 1, 2, 8);
+        HXQ_RWS(4, 2, 1, 8);
+        HXQ_RWS(4, 3, 1, 8);
+        HXQ_RWS(4, 5, 1, 8);
+    }
+#undef HXQ_RWS
+    HXQ_REQUIRE(false, "no such few-row plan");
+}
+
+}  // namespace rw
+}  // namespace hxq

@@ -1,0 +1,73 @@
+"""hxq_prefill_gemm on few rows of X (hxq_rows.h) at the edges of its tiles: 16-row tiles of X
+and W, 64-row blocks, one 64-column step up to several per wave, runs of 1, 2, 3 and 5 subtiles,
+every affine group layout and index format, sidecars denser than the 32 entries a row group
+holds per iteration."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helix_substrate import _hxq
+from test_gpu_formats import FMTS, _case, _dev, _grp, _maxrel, _wide_layer
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(dev, fmt, m, out, inp, G, xdt, density=0.001):
+    if fmt == _hxq.FMT_SCALAR_U16:
+        mod, W, Wf = _wide_layer(out, inp, 3000, seed=m + out, group_size=G, density=density, fma=True)
+        raw, cb, aff, gp, gk, gv = _dev(dev, mod.indices, mod.codebook, mod._affine_t,
+                                        mod._sc_grp_ptr, mod._sc_grp_key, mod._sc_grp_val)
+    elif fmt == _hxq.FMT_SCALAR:
+        from helix_substrate import synth
+        L = synth.make_layer_np(out, inp, seed=m + inp, group_size=G, density=density)
+        args = (L["indices"], L["codebook"], L["group_scale"], L["group_offset"], G,
+                L["sidecar_positions"], L["sidecar_values"])
+        W, Wf = oracle.reconstruct(*args), oracle.reconstruct(*args, fma=True)
+        aff = np.ascontiguousarray(np.stack([L["group_scale"].T, L["group_offset"].T], axis=-1))
+        raw, cb, aff = _dev(dev, L["indices"], L["codebook"], aff)
+        gp, gk, gv = _grp(dev, L["sidecar_positions"], L["sidecar_values"], out, inp)
+    else:
+        raw, cb, s, o, pos, val, W, _ = _case(fmt, out, inp, G=G, seed=m + inp)
+        Wf = W if s is None else _case(fmt, out, inp, G=G, seed=m + inp, fma=True)[6]
+        aff = None if s is None else np.ascontiguousarray(np.stack([s.T, o.T], axis=-1))
+        raw, cb, aff = _dev(dev, raw, cb, aff)
+        gp, gk, gv = _grp(dev, pos, val, out, inp)
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, inp, generator=g).to(xdt)
+    bias = torch.randn(out, generator=g) * 0.1
+    print(f"rows fmt={fmt} m={m} out={out} in={inp} G={G} x={xdt}", flush=True)
+    args = (x.to(dev), raw, cb, aff, G, gp, gk, gv, bias.to(dev))
+    y = _hxq.prefill_gemm(*args, out_dtype=torch.float32, fmt=fmt, out_features=out)
+    xf = x.float().numpy()
+    # fp32 X: order of fp32 sums only; 16-bit X: likewise, once W is rounded as the operands are
+    Wr, bar = (W, 1e-5) if xdt == torch.float32 else (torch.from_numpy(Wf).to(xdt).float().numpy(), 2e-5)
+    rel = _maxrel(y.cpu().numpy(), oracle.linear_np(xf, Wr, bias.numpy()))
+    assert rel <= bar, rel
+    assert torch.equal(_hxq.prefill_gemm(*args, out_dtype=torch.float32, fmt=fmt, out_features=out), y)
+    y16 = _hxq.prefill_gemm(*args, fmt=fmt, out_features=out)
+    assert torch.equal(y16, y.to(xdt))   # the same sums, rounded once
+
+
+@pytest.mark.parametrize("m,out,inp,G", [
+    (1, 16, 64, 64), (5, 15, 64, 16), (16, 17, 1088, 32), (17, 81, 1024, 128), (33, 300, 2048, 128),
+    (64, 4100, 448, 64), (65, 530, 576, 48), (130, 100, 4160, 64), (16, 12300, 320, 64),
+    (40, 20500, 192, 64), (48, 256, 8256, 64),
+])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+def test_rows_edges(dev, m, out, inp, G, xdt):
+    _check(dev, _hxq.FMT_SCALAR, m, out, inp, G, xdt)
+
+
+@pytest.mark.parametrize("fmt", FMTS + [_hxq.FMT_SCALAR_U16])
+@pytest.mark.parametrize("m,out,inp", [(7, 48, 128), (31, 5000, 640), (63, 258, 1152)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
+def test_rows_formats(dev, fmt, m, out, inp, xdt):
+    _check(dev, fmt, m, out, inp, 128 if inp % 128 == 0 else 64, xdt)
+
+
+@pytest.mark.parametrize("m,out,inp", [(9, 130, 512), (20, 8200, 256)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+def test_rows_dense_sidecar(dev, m, out, inp, xdt):
+    """5 % of the weights: some 200 entries per row group and step."""
+    _check(dev, _hxq.FMT_SCALAR, m, out, inp, 128, xdt, density=0.05)
