@@ -1,0 +1,63 @@
+"""The encoder's kernels at the edges of their blocks and trees, bit for bit against the oracle:
+assignment for codebook sizes around powers of two (levels of the search tree), ties, infinities
+and unaligned inputs; k-means whose sort and scatter blocks, cluster sizes and pairwise trees end
+just before, at and just after a boundary."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helix_substrate import _hxq
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 127, 128, 255, 256, 257, 1000, 4095, 4096])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_assign_codebook_sizes(dev, k, offset):
+    rs = np.random.RandomState(k)
+    cb = np.sort(rs.standard_normal(k).astype(np.float32))
+    cb[k // 3:k // 2] = cb[k // 3] if k > 2 else cb[k // 3:k // 2]   # a run of equal entries
+    mid = ((cb[1:] + cb[:-1]) / 2).astype(np.float32)
+    x = np.concatenate([rs.standard_normal(5003).astype(np.float32) * 2, cb, mid,
+                        np.float32([np.inf, -np.inf, np.nan, 0.0, -0.0, 3e38, -3e38, 1e-40])])
+    print(f"assign k={k} offset={offset} n={x.size}", flush=True)
+    buf = torch.zeros(x.size + 4, device=dev)
+    buf[offset:offset + x.size] = torch.from_numpy(x).to(dev)   # offset 1: no 16-byte alignment
+    got = _hxq.assign_nearest(buf[offset:offset + x.size], torch.from_numpy(cb).to(dev))
+    got = got.cpu().numpy().astype(np.int64) & 0xffff
+    np.testing.assert_array_equal(got, oracle.assign_nearest_np(x, cb).astype(np.int64))
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (7, 3), (2047, 256), (2048, 64), (2049, 256), (4096, 5),
+                                 (8192, 1), (8193, 1), (8191 + 129, 2), (70001, 300)])
+def test_kmeans_block_edges(dev, n, k):
+    rs = np.random.RandomState(n)
+    data = rs.standard_normal(n).astype(np.float32)
+    if n > 100:
+        data[rs.randint(0, n, n // 5)] = np.float32([-0.0, 0.0, 0.5])[rs.randint(0, 3, n // 5)]
+    print(f"kmeans n={n} k={k}", flush=True)
+    cb, asg, it = _hxq.kmeans_1d(torch.from_numpy(data).to(dev), k, 10, 0.001)
+    if cb.numel() <= 256:
+        cb_o, asg_o, it_o = oracle.kmeans_np(data, k)
+        np.testing.assert_array_equal(asg.cpu().numpy(), asg_o)
+        assert it == it_o
+    else:   # integer cluster ids (the oracle's are uint8)
+        from helix_substrate.hxq_encoder import _simple_kmeans
+        cb_o, asg_o = _simple_kmeans(data, k)
+        np.testing.assert_array_equal(asg.cpu().numpy().view(np.uint16), asg_o)
+    np.testing.assert_array_equal(cb.cpu().numpy(), cb_o)
+
+
+@pytest.mark.parametrize("sizes", [(63, 64, 65, 127, 128, 129, 130, 255, 256, 257), (8191, 8192, 8193, 16385)])
+def test_kmeans_cluster_sizes(dev, sizes):
+    """Well separated clusters of given sizes: every shape of the pairwise tree."""
+    rs = np.random.RandomState(5)
+    data = np.concatenate([10.0 * j + rs.standard_normal(m) for j, m in enumerate(sizes)]).astype(np.float32)
+    data = data[rs.permutation(data.size)]
+    print(f"kmeans sizes={sizes}", flush=True)
+    cb, asg, it = _hxq.kmeans_1d(torch.from_numpy(data).to(dev), len(sizes), 10, 0.001)
+    cb_o, asg_o, it_o = oracle.kmeans_np(data, len(sizes))
+    np.testing.assert_array_equal(cb.cpu().numpy(), cb_o)
+    np.testing.assert_array_equal(asg.cpu().numpy(), asg_o)
+    assert it == it_o
