@@ -203,6 +203,13 @@ constexpr int kWaves = kThreads / kWave;
 constexpr int kRounds = kPer / kThreads;    // elements per lane
 constexpr int kDigits = 256;
 
+// Waits until this wave's stores and atomics are done.  Where they are
+// device-scope atomics (performed past the XCD's own L2) and are read back by
+// device-scope atomic loads, this orders them before a counter that another
+// block looks at; a device-scope fence would also write the L2 back, for every
+// wave that meets it (the select passes: 150 us with it, 30 without).
+__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Radix digit of the sort keys; the first pass makes the keys from x.
 struct DigitSrc {
     const float *x;        // first pass, else null
@@ -545,13 +552,12 @@ __global__ __launch_bounds__(kThreads) void km_sum_kernel(const float *sorted_va
     if (threadIdx.x == 0) {
         const float mean = c == 0 ? cb[j] : sum / static_cast<float>(c);
         __hip_atomic_store(&means[j], mean, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __threadfence();
+        wait_vmem();
         s_flag = atomicAdd(arrived, 1) == k - 1;
     }
     __syncthreads();
     if (!s_flag) return;
     // the last cluster's block: movement, convergence, the new codebook
-    __threadfence();
     float mx = 0.f;
     int nan = 0;
     for (int q = threadIdx.x; q < k; q += kThreads) {
@@ -588,121 +594,230 @@ __global__ __launch_bounds__(kThreads) void km_sum_kernel(const float *sorted_va
 // ---------------------------------------------------------------------------
 constexpr int kSelMax = 4;
 
+// Digits of 11, 11 and 10 bits of the sort key, from the top.
+constexpr int kSelBins = 2048;
+__host__ __device__ constexpr int sel_shift(int pass) { return pass == 0 ? 21 : pass == 1 ? 10 : 0; }
+
 struct SelState {
     uint32_t prefix[kSelMax];  // key bits fixed so far
     uint32_t rank[kSelMax];    // rank within the keys matching prefix
-    uint32_t hist[kSelMax][256];
+    uint32_t hist[kSelMax][kSelBins];
     int32_t nan_count;
-    int32_t pad_;
+    int32_t arrived;
 };
 
-__global__ __launch_bounds__(kThreads) void select_hist_kernel(const float *x, int64_t n, int m,
-                                                               int shift, SelState *st) {
-    __shared__ uint32_t h[kSelMax][256];
-    for (int i = threadIdx.x; i < kSelMax * 256; i += kThreads) (&h[0][0])[i] = 0;
-    __syncthreads();
+constexpr int kSelThreads = 1024;
+// One pass: a histogram of the digit over the keys that match a rank's
+// prefix, and in the last block to finish, the digit each rank falls into.
+// Ranks with one prefix share a histogram (all of them in the first pass,
+// neighbours usually to the end).  Bound by reading x (16 bytes a lane;
+// 22.5M values: 31 us for the first pass, 25 us for the others, whose matches
+// are few; blocks of 4 waves, which keep half as many loads in flight, 47;
+// four 8-bit passes that counted every rank for itself 69 us each, and 15 us
+// for one thread a rank picking the digit).
+__global__ __launch_bounds__(kSelThreads) void select_pass_kernel(const float *x, int64_t n, int m, int pass,
+                                                               int vec, SelState *st, float *out) {
+    __shared__ uint32_t h[kSelMax][kSelBins];
+    __shared__ int s_last;
+    __shared__ int s_w[kSelThreads / kWave];
+    const int shift = sel_shift(pass);
+    const uint32_t hi_mask = pass == 0 ? 0u : pass == 1 ? 0xffffffffu << 21 : 0xffffffffu << 10;
     uint32_t pre[kSelMax];
-    for (int r = 0; r < m; ++r) pre[r] = st->prefix[r];
-    const uint32_t hi_mask = shift >= 24 ? 0u : (0xffffffffu << (shift + 8));
+    int slot[kSelMax];   // the first rank with this prefix
+#pragma unroll
+    for (int r = 0; r < kSelMax; ++r) {
+        pre[r] = st->prefix[min(r, m - 1)];
+        slot[r] = r;
+#pragma unroll
+        for (int q = kSelMax - 1; q >= 0; --q)
+            if (q < r && pre[q] == pre[r]) slot[r] = q;
+    }
+    for (int i = threadIdx.x; i < kSelMax * kSelBins; i += kSelThreads) (&h[0][0])[i] = 0;
+    __syncthreads();
     int32_t nans = 0;
-    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * kThreads) {
-        const uint32_t key = sort_key(x[i]);
-        if (shift == 24 && key == 0xffffffffu) ++nans;
-        const uint32_t d = (key >> shift) & 0xffu;
-        for (int r = 0; r < m; ++r)
-            if ((key & hi_mask) == (pre[r] & hi_mask)) atomicAdd(&h[r][d], 1u);
+    auto count = [&](float v) {
+        const uint32_t key = sort_key(v);
+        if (pass == 0 && key == 0xffffffffu) ++nans;
+        const uint32_t d = (key >> shift) & (pass == 2 ? 1023u : 2047u);
+#pragma unroll
+        for (int r = 0; r < kSelMax; ++r)
+            if (r < m && slot[r] == r && ((key ^ pre[r]) & hi_mask) == 0) atomicAdd(&h[r][d], 1u);
+    };
+    // 8 consecutive values a thread and round
+    for (int64_t i0 = (blockIdx.x * (int64_t)kSelThreads + threadIdx.x) * 8; i0 < n;
+         i0 += (int64_t)gridDim.x * kSelThreads * 8) {
+        if (vec && i0 + 8 <= n) {
+            const float4 a = *reinterpret_cast<const float4 *>(x + i0);
+            const float4 b = *reinterpret_cast<const float4 *>(x + i0 + 4);
+            count(a.x); count(a.y); count(a.z); count(a.w);
+            count(b.x); count(b.y); count(b.z); count(b.w);
+        } else {
+            for (int q = 0; q < 8; ++q)
+                if (i0 + q < n) count(x[i0 + q]);
+        }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < m * 256; i += kThreads) {
+    for (int i = threadIdx.x; i < m * kSelBins; i += kSelThreads) {
         const uint32_t v = (&h[0][0])[i];
-        if (v) atomicAdd(&st->hist[i / 256][i % 256], v);
+        if (v) atomicAdd(&st->hist[i / kSelBins][i % kSelBins], v);
     }
-    if (shift == 24 && nans) atomicAdd(&st->nan_count, nans);
-}
-
-__global__ void select_pick_kernel(int m, int shift, SelState *st, float *out) {
-    const int r = threadIdx.x;
-    if (r < m) {
-        uint32_t rank = st->rank[r];
-        int d = 0;
-        for (; d < 255; ++d) {
-            const uint32_t c = st->hist[r][d];
-            if (rank < c) break;
-            rank -= c;
+    if (pass == 0 && nans) atomicAdd(&st->nan_count, nans);
+    wait_vmem();
+    __syncthreads();
+    if (threadIdx.x == 0) s_last = atomicAdd(&st->arrived, 1) == static_cast<int>(gridDim.x) - 1;
+    __syncthreads();
+    if (!s_last) return;
+    // the last block: rank r falls into the first bin whose running count
+    // passes it; each thread holds PT consecutive bins
+    constexpr int PT = kSelBins / kSelThreads;
+    for (int r = 0; r < m; ++r) {
+        uint32_t c[PT];
+        uint32_t sum = 0;
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
+            c[q] = __hip_atomic_load(&st->hist[slot[r]][threadIdx.x * PT + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sum += c[q];
         }
-        st->prefix[r] |= static_cast<uint32_t>(d) << shift;
-        st->rank[r] = rank;
-        for (int i = 0; i < 256; ++i) st->hist[r][i] = 0;
-        if (shift == 0) out[r] = key_float(st->prefix[r]);
+        const uint32_t inc = static_cast<uint32_t>(wave_scan(static_cast<int>(sum)));
+        if ((threadIdx.x & 63) == 63) s_w[threadIdx.x / kWave] = static_cast<int>(inc);
+        __syncthreads();
+        uint32_t base = inc - sum;
+        for (int w = 0; w < static_cast<int>(threadIdx.x / kWave); ++w) base += static_cast<uint32_t>(s_w[w]);
+        const uint32_t rank = st->rank[r];
+        if (rank >= base && rank - base < sum) {   // one thread
+            uint32_t left = rank - base;
+            int d = 0;
+#pragma unroll
+            for (int q = 0; q < PT; ++q) {
+                if (d == q && left >= c[q]) {
+                    left -= c[q];
+                    ++d;
+                }
+            }
+            const uint32_t p = pre[r] | static_cast<uint32_t>(threadIdx.x * PT + d) << shift;
+            st->prefix[r] = p;
+            h[0][r] = left;      // (st->rank[r] is still being read)
+            if (pass == 2) out[r] = key_float(p);
+        }
+        __syncthreads();
     }
+    if (threadIdx.x < m) st->rank[threadIdx.x] = h[0][threadIdx.x];
+    for (int i = threadIdx.x; i < m * kSelBins; i += kSelThreads) st->hist[i / kSelBins][i % kSelBins] = 0;
+    if (threadIdx.x == 0) st->arrived = 0;
 }
 
 __global__ void select_init_kernel(const int64_t *ranks, int m, SelState *st) {
-    for (int i = threadIdx.x; i < kSelMax * 256; i += blockDim.x) (&st->hist[0][0])[i] = 0;
+    for (int i = threadIdx.x; i < kSelMax * kSelBins; i += blockDim.x) (&st->hist[0][0])[i] = 0;
     if (threadIdx.x < kSelMax) {
         st->prefix[threadIdx.x] = 0;
         st->rank[threadIdx.x] = threadIdx.x < m ? static_cast<uint32_t>(ranks[threadIdx.x]) : 0;
     }
-    if (threadIdx.x == 0) st->nan_count = 0;
-}
-
-// outliers: x < lo or x > hi, positions ascending (two passes)
-__global__ __launch_bounds__(kThreads) void outlier_count_kernel(const float *x, int64_t n, int64_t per,
-                                                                 const float *lohi, int32_t *blk) {
-    __shared__ int32_t s;
-    if (threadIdx.x == 0) s = 0;
-    __syncthreads();
-    const float lo = lohi[0], hi = lohi[1];
-    const int64_t a = blockIdx.x * per, b = min(n, a + per);
-    int32_t c = 0;
-    for (int64_t i = a + threadIdx.x; i < b; i += kThreads) {
-        const float v = x[i];
-        c += (v < lo) | (v > hi);
-    }
-    atomicAdd(&s, c);
-    __syncthreads();
-    if (threadIdx.x == 0) blk[blockIdx.x] = s;
-}
-
-__global__ void outlier_scan_kernel(int32_t *blk, int nblk, int64_t *total) {
     if (threadIdx.x == 0) {
-        int64_t s = 0;
-        for (int b = 0; b < nblk; ++b) { const int32_t c = blk[b]; blk[b] = static_cast<int32_t>(s); s += c; }
-        *total = s;
+        st->nan_count = 0;
+        st->arrived = 0;
     }
 }
 
-__global__ __launch_bounds__(kThreads) void outlier_write_kernel(const float *x, int64_t n, int64_t per,
-                                                                 const float *lohi, const int32_t *blk,
-                                                                 int64_t cap, int64_t *pos, float *val) {
-    constexpr int W = kThreads / kWave;
-    __shared__ int32_t wsum[W];
-    __shared__ int32_t base;
-    if (threadIdx.x == 0) base = blk[blockIdx.x];
+// Outliers: x < lo or x > hi, positions ascending, in two passes over x.  A
+// wave owns kChunk consecutive values, 256 a round (four consecutive ones a
+// lane); the chunks' counts are scanned in between, so that no wave waits for
+// another.  Bound by reading x: 22.5M values 16 us a pass (65536-value blocks
+// with a block-wide scan per 256 values: 80 and 127 us, 38 us for one thread
+// scanning the blocks).
+constexpr int kChunk = 4096;
+
+__device__ __forceinline__ float4 load4(const float *x, int64_t i, int64_t n, int vec) {
+    if (vec && i + 4 <= n) return *reinterpret_cast<const float4 *>(x + i);
+    const float none = __uint_as_float(0x7fc00000u);   // NaN: never an outlier
+    return make_float4(i < n ? x[i] : none, i + 1 < n ? x[i + 1] : none, i + 2 < n ? x[i + 2] : none,
+                       i + 3 < n ? x[i + 3] : none);
+}
+
+__global__ __launch_bounds__(kThreads) void outlier_count_kernel(const float *x, int64_t n, int64_t chunks, int vec,
+                                                                 const float *lohi, int64_t *cnt) {
+    const int lane = threadIdx.x & 63;
+    const int64_t ch = blockIdx.x * (int64_t)kWaves + threadIdx.x / kWave;
+    if (ch >= chunks) return;
     const float lo = lohi[0], hi = lohi[1];
-    const int lane = threadIdx.x & 63, w = threadIdx.x / kWave;
-    const int64_t a = blockIdx.x * per, b = min(n, a + per);
-    for (int64_t c0 = a; c0 < b; c0 += kThreads) {
-        const int64_t i = c0 + threadIdx.x;
-        const float v = i < b ? x[i] : 0.f;
-        const bool hit = i < b && ((v < lo) | (v > hi));
-        const uint64_t mask = __ballot(hit);
-        const int r = __popcll(mask & ((1ull << lane) - 1ull));
-        if (lane == 0) wsum[w] = __popcll(mask);
+    int c = 0;
+#pragma unroll 8
+    for (int r = 0; r < kChunk / 256; ++r) {
+        const float4 v = load4(x, ch * kChunk + r * 256 + lane * 4, n, vec);
+        c += (v.x < lo) | (v.x > hi);
+        c += (v.y < lo) | (v.y > hi);
+        c += (v.z < lo) | (v.z > hi);
+        c += (v.w < lo) | (v.w > hi);
+    }
+    c = __builtin_amdgcn_readlane(wave_scan(c), 63);
+    if (lane == 0) cnt[ch] = c;
+}
+
+// cnt[c] -> outliers in chunks before c; *total = all of them
+__global__ __launch_bounds__(1024) void outlier_scan_kernel(int64_t *cnt, int64_t chunks, int64_t *total) {
+    __shared__ int s_w[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int64_t base = 0;
+    for (int64_t c0 = 0; c0 < chunks; c0 += 4096) {
+        int v[4], sum = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t c = c0 + threadIdx.x * 4 + q;
+            v[q] = c < chunks ? static_cast<int>(cnt[c]) : 0;
+            sum += v[q];
+        }
+        const int inc = wave_scan(sum);
+        if (lane == 63) s_w[w] = inc;
         __syncthreads();
-        if (hit) {
-            int64_t p = base + r;
-            for (int ww = 0; ww < w; ++ww) p += wsum[ww];
-            if (p < cap) { pos[p] = i; val[p] = v; }
+        int64_t s = base + inc - sum;
+        for (int q = 0; q < 16; ++q) {
+            if (q < w) s += s_w[q];
+            base += s_w[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t c = c0 + threadIdx.x * 4 + q;
+            if (c < chunks) cnt[c] = s;
+            s += v[q];
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            int32_t s = 0;
-            for (int ww = 0; ww < W; ++ww) s += wsum[ww];
-            base += s;
+    }
+    if (threadIdx.x == 0) *total = base;
+}
+
+__global__ __launch_bounds__(kThreads) void outlier_write_kernel(const float *x, int64_t n, int64_t chunks, int vec,
+                                                                 const float *lohi, const int64_t *cnt,
+                                                                 int64_t cap, int64_t *pos, float *val) {
+    const int lane = threadIdx.x & 63;
+    const int64_t ch = blockIdx.x * (int64_t)kWaves + threadIdx.x / kWave;
+    if (ch >= chunks) return;
+    const float lo = lohi[0], hi = lohi[1];
+    int64_t base = cnt[ch];
+#pragma unroll 8
+    for (int r = 0; r < kChunk / 256; ++r) {
+        const int64_t i = ch * kChunk + r * 256 + lane * 4;
+        const float4 v = load4(x, i, n, vec);
+        const float e[4] = {v.x, v.y, v.z, v.w};
+        bool hit[4];
+        int c = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            hit[q] = (e[q] < lo) | (e[q] > hi);
+            c += hit[q];
         }
-        __syncthreads();
+        if (__ballot(c != 0) == 0) continue;   // wave-uniform
+        const int inc = wave_scan(c);
+        int64_t p = base + inc - c;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (hit[q]) {
+                if (p < cap) {
+                    pos[p] = i + q;
+                    val[p] = e[q];
+                }
+                ++p;
+            }
+        }
+        base += __builtin_amdgcn_readlane(inc, 63);
     }
 }
 
@@ -728,12 +843,49 @@ __global__ __launch_bounds__(kThreads) void zero_u32_kernel(uint32_t *p, int64_t
         p[i] = 0u;
 }
 
-__device__ __forceinline__ double wave_sum_f64(double v) {
+// v + the value of the lane the moves of its two halves name
+template <int CTRL>
+__device__ __forceinline__ double dpp_add_f64(double v) {
 #pragma clang fp contract(off)
-    for (int m = 32; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, kWave);
-    return v;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xf, 0xf, false);
+    return v + __longlong_as_double(static_cast<long long>(hi) << 32 | static_cast<unsigned int>(lo));
 }
 
+__device__ __forceinline__ double swap_add_f64(double p, double q, bool by32) {
+#pragma clang fp contract(off)
+    const long long a = __double_as_longlong(p), b = __double_as_longlong(q);
+    const unsigned int al = static_cast<unsigned int>(a), ah = static_cast<unsigned int>(a >> 32);
+    const unsigned int bl = static_cast<unsigned int>(b), bh = static_cast<unsigned int>(b >> 32);
+    const auto lo = by32 ? __builtin_amdgcn_permlane32_swap(al, bl, false, false)
+                         : __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto hi = by32 ? __builtin_amdgcn_permlane32_swap(ah, bh, false, false)
+                         : __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    return __longlong_as_double(static_cast<long long>(hi[0]) << 32 | lo[0]) +
+           __longlong_as_double(static_cast<long long>(hi[1]) << 32 | lo[1]);
+}
+
+// Wave sums of four values, each in the order of an xor butterfly 32, 16, ...,
+// 1 and without LDS: a lane swap halves two values against each other (the
+// lower lanes go on with the first, the upper ones with the second), so after
+// the steps 32 and 16 one register holds all four, a row of 16 lanes each:
+// v[0], v[2], v[1], v[3].  Within a row a rotation by 8, 4, 2 and 1 stands for
+// the xor: after each step the values repeat with that period.
+__device__ __forceinline__ double wave_sum4_f64(const double (&v)[4]) {
+    const double p = swap_add_f64(v[0], v[1], true), q = swap_add_f64(v[2], v[3], true);
+    double r = swap_add_f64(p, q, false);
+    r = dpp_add_f64<0x128>(r);  // row_ror:8
+    r = dpp_add_f64<0x124>(r);
+    r = dpp_add_f64<0x122>(r);
+    return dpp_add_f64<0x121>(r);
+}
+
+// A wave fits kFitUnits consecutive groups, their loads all requested first.
+// 11008 x 2048 weights in groups of 128: 69 us, bound by the fp64 additions
+// (each sum by itself over the wave 90; by LDS permutes, one group per wave,
+// 120).
+constexpr int kFitUnits = 4;
 template <typename IT, int KM>
 __global__ __launch_bounds__(kThreads) void affine_fit_kernel(const float *w, const IT *idx,
                                                               const float *cb, int k, int64_t rows,
@@ -745,42 +897,54 @@ __global__ __launch_bounds__(kThreads) void affine_fit_kernel(const float *w, co
     for (int j = threadIdx.x; j < KM; j += kThreads) s_cb[j] = j < k ? cb[j] : 0.f;
     __syncthreads();
     const int lane = threadIdx.x & 63;
-    const int64_t ngroups = cols / group;
-    const int64_t unit = blockIdx.x * (int64_t)(kThreads / kWave) + threadIdx.x / kWave;
-    if (unit >= rows * ngroups) return;
-    const int64_t r = unit / ngroups, g = unit % ngroups;
-    const int64_t base = r * cols + g * group;
-    double sc = 0.0, sw = 0.0, scc = 0.0, scw = 0.0, sn = 0.0;
-    for (int t = lane; t < group; t += kWave) {
-        const int64_t e = base + t;
-        const bool skip = bits && ((bits[e >> 5] >> (e & 31)) & 1u);
-        if (!skip) {
-            // an index past the table (a caller error) reads a zero entry, in bounds
-            const double c = static_cast<double>(s_cb[min(static_cast<int>(idx[e]), KM - 1)]);
-            const double x = static_cast<double>(w[e]);
-            sc = sc + c;
-            sw = sw + x;
-            scc = scc + c * c;
-            scw = scw + c * x;
-            sn = sn + 1.0;
+    const int64_t ngroups = cols / group, units = rows * ngroups;
+    const int64_t u0 = (blockIdx.x * (int64_t)kWaves + threadIdx.x / kWave) * kFitUnits;
+    double sc[kFitUnits], sw[kFitUnits], scc[kFitUnits], scw[kFitUnits], sn[kFitUnits];
+#pragma unroll
+    for (int u = 0; u < kFitUnits; ++u) sc[u] = sw[u] = scc[u] = scw[u] = sn[u] = 0.0;
+    for (int t = lane; t - lane < group; t += kWave) {
+        float x[kFitUnits];
+        int id[kFitUnits];
+        bool use[kFitUnits];
+#pragma unroll
+        for (int u = 0; u < kFitUnits; ++u) {
+            // the groups of a row, and the rows, follow each other in memory
+            const int64_t e = (u0 + u) * group + t;
+            use[u] = u0 + u < units && t < group;
+            x[u] = use[u] ? w[e] : 0.f;
+            id[u] = use[u] ? idx[e] : 0;
+            if (bits && use[u]) use[u] = !((bits[e >> 5] >> (e & 31)) & 1u);
+        }
+#pragma unroll
+        for (int u = 0; u < kFitUnits; ++u) {
+            if (use[u]) {
+                // an index past the table (a caller error) reads a zero entry, in bounds
+                const double c = static_cast<double>(s_cb[min(id[u], KM - 1)]);
+                const double v = static_cast<double>(x[u]);
+                sc[u] = sc[u] + c;
+                sw[u] = sw[u] + v;
+                scc[u] = scc[u] + c * c;
+                scw[u] = scw[u] + c * v;
+            }
+            sn[u] += static_cast<double>(__popcll(__ballot(use[u])));  // (exact in any order)
         }
     }
-    sc = wave_sum_f64(sc);
-    sw = wave_sum_f64(sw);
-    scc = wave_sum_f64(scc);
-    scw = wave_sum_f64(scw);
-    sn = wave_sum_f64(sn);
-    if (lane == 0) {
+    // row r of 16 lanes holds group {0, 2, 1, 3}[r]; its first lane solves it
+    const double a = wave_sum4_f64(sc), b = wave_sum4_f64(sw), aa = wave_sum4_f64(scc), ab = wave_sum4_f64(scw);
+    const int row = lane >> 4;
+    const int u = (row >> 1) | ((row & 1) << 1);
+    const double n = u == 0 ? sn[0] : u == 1 ? sn[1] : u == 2 ? sn[2] : sn[3];
+    if ((lane & 15) == 0 && u0 + u < units) {
         double s = 1.0, o = 0.0;
-        const double det = sn * scc - sc * sc;
-        if (sn >= 2.0 && det > 0.0) {
-            s = (sn * scw - sc * sw) / det;
-            o = (sw - s * sc) / sn;
-        } else if (sn > 0.0) {
-            o = (sw - sc) / sn;
+        const double det = n * aa - a * a;
+        if (n >= 2.0 && det > 0.0) {
+            s = (n * ab - a * b) / det;
+            o = (b - s * a) / n;
+        } else if (n > 0.0) {
+            o = (b - a) / n;
         }
-        scale[r * ngroups + g] = static_cast<float>(s);
-        offset[r * ngroups + g] = static_cast<float>(o);
+        scale[u0 + u] = static_cast<float>(s);
+        offset[u0 + u] = static_cast<float>(o);
     }
 }
 
@@ -1201,11 +1365,13 @@ extern "C" int hxq_select_f32(const float *x, int64_t n, const int64_t *ranks, i
     SelState *st = static_cast<SelState *>(workspace);
     hipLaunchKernelGGL(select_init_kernel, dim3(1), dim3(256), 0, stream, ranks, m, st);
     HXQ_LAUNCH_CHECK();
-    const int g = std::min(grid_for(n), 2048);
-    for (int shift = 24; shift >= 0; shift -= 8) {
-        hipLaunchKernelGGL(select_hist_kernel, dim3(g), dim3(kThreads), 0, stream, x, n, m, shift, st);
-        HXQ_LAUNCH_CHECK();
-        hipLaunchKernelGGL(select_pick_kernel, dim3(1), dim3(64), 0, stream, m, shift, st, values);
+    // two blocks of 16 waves per CU: the histograms (32 KB of LDS) are added up
+    // once per block
+    const int64_t blocks = (n + kSelThreads * 8 - 1) / (kSelThreads * 8);
+    const dim3 grid(static_cast<uint32_t>(std::min<int64_t>(blocks, 2 * device_cu_count())));
+    const int vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    for (int pass = 0; pass < 3; ++pass) {
+        hipLaunchKernelGGL(select_pass_kernel, grid, dim3(kSelThreads), 0, stream, x, n, m, pass, vec, st, values);
         HXQ_LAUNCH_CHECK();
     }
     if (nan_count)
@@ -1214,8 +1380,7 @@ extern "C" int hxq_select_f32(const float *x, int64_t n, const int64_t *ranks, i
 }
 
 extern "C" int64_t hxq_outliers_workspace_bytes(int64_t n) {
-    const int64_t nblk = (n + 65535) / 65536;
-    return 4 * std::max<int64_t>(nblk, 1) + 64;
+    return 8 * std::max<int64_t>((n + kChunk - 1) / kChunk, 1) + 64;
 }
 
 extern "C" int hxq_outliers_f32(const float *x, int64_t n, const float *lohi, int64_t capacity,
@@ -1226,16 +1391,19 @@ extern "C" int hxq_outliers_f32(const float *x, int64_t n, const float *lohi, in
                 "bad arguments");
     HXQ_REQUIRE(n >= 1 && capacity >= 0, "bad sizes");
     HXQ_REQUIRE(workspace_bytes >= hxq_outliers_workspace_bytes(n), "workspace too small");
-    const int64_t per = 65536;
-    const int nblk = static_cast<int>((n + per - 1) / per);
-    int32_t *blk = static_cast<int32_t *>(workspace);
-    hipLaunchKernelGGL(outlier_count_kernel, dim3(nblk), dim3(kThreads), 0, stream, x, n, per, lohi, blk);
+    const int64_t chunks = (n + kChunk - 1) / kChunk;
+    const dim3 grid(static_cast<uint32_t>((chunks + kWaves - 1) / kWaves));
+    HXQ_REQUIRE((chunks + kWaves - 1) / kWaves < (int64_t{1} << 31), "n too large");
+    HXQ_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 7u) == 0, "workspace must be 8-byte aligned");
+    const int vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    int64_t *cnt = static_cast<int64_t *>(workspace);
+    hipLaunchKernelGGL(outlier_count_kernel, grid, dim3(kThreads), 0, stream, x, n, chunks, vec, lohi, cnt);
     HXQ_LAUNCH_CHECK();
-    hipLaunchKernelGGL(outlier_scan_kernel, dim3(1), dim3(64), 0, stream, blk, nblk, count);
+    hipLaunchKernelGGL(outlier_scan_kernel, dim3(1), dim3(1024), 0, stream, cnt, chunks, count);
     HXQ_LAUNCH_CHECK();
     if (capacity > 0) {
-        hipLaunchKernelGGL(outlier_write_kernel, dim3(nblk), dim3(kThreads), 0, stream, x, n, per, lohi,
-                           blk, capacity, positions, values);
+        hipLaunchKernelGGL(outlier_write_kernel, grid, dim3(kThreads), 0, stream, x, n, chunks, vec, lohi, cnt,
+                           capacity, positions, values);
         HXQ_LAUNCH_CHECK();
     }
     return HXQ_OK;
@@ -1270,7 +1438,7 @@ static int affine_fit_impl(const float *w, const IT *indices, const float *codeb
         HXQ_LAUNCH_CHECK();
     }
     const int64_t units = rows * (cols / group_size);
-    const int64_t per_block = kThreads / kWave;
+    const int64_t per_block = kWaves * kFitUnits;
     const int64_t blocks = (units + per_block - 1) / per_block;
     HXQ_REQUIRE(blocks < (int64_t{1} << 31), "too many groups");
     hipLaunchKernelGGL((affine_fit_kernel<IT, KM>), dim3(static_cast<uint32_t>(blocks)), dim3(kThreads),

@@ -61,3 +61,43 @@ def test_kmeans_cluster_sizes(dev, sizes):
     np.testing.assert_array_equal(cb.cpu().numpy(), cb_o)
     np.testing.assert_array_equal(asg.cpu().numpy(), asg_o)
     assert it == it_o
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 4095, 4096, 4097, 8191, 16389, 262147])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+def test_select_and_outlier_edges(dev, n, offset):
+    """Order statistics and outliers around the chunks' and blocks' ends, at every alignment,
+    with values that share their upper key bits."""
+    rs = np.random.RandomState(n + offset)
+    x = rs.standard_normal(n).astype(np.float32)
+    x[rs.randint(0, n, max(1, n // 3))] = np.float32(1.0) + rs.randint(0, 4, max(1, n // 3)) * np.float32(2 ** -23)
+    x[rs.randint(0, n)] = -np.inf
+    print(f"select n={n} offset={offset}", flush=True)
+    buf = torch.zeros(n + 4, device=dev)
+    buf[offset:offset + n] = torch.from_numpy(x).to(dev)
+    d = buf[offset:offset + n]
+    ranks = [0, n // 2, min(n - 1, n // 2 + 1), n - 1]
+    vals, nans = _hxq.select_f32(d, ranks)
+    np.testing.assert_array_equal(vals.cpu().numpy(), np.sort(x)[ranks])
+    assert nans == 0
+    for lo, hi in ((-1.5, 1.5), (-np.inf, np.inf), (0.0, 0.0)):
+        pos, val = _hxq.outliers_f32(d, lo, hi)
+        want = np.where((x < np.float32(lo)) | (x > np.float32(hi)))[0]
+        np.testing.assert_array_equal(pos.cpu().numpy(), want)
+        np.testing.assert_array_equal(val.cpu().numpy(), x[want])
+
+
+@pytest.mark.parametrize("rows,cols,G", [(1, 16, 16), (3, 96, 96), (5, 260, 52), (7, 640, 128), (2, 384, 1)])
+def test_affine_fit_edges(dev, rows, cols, G):
+    """Group counts that are no multiple of a wave's four, groups below, at and above a wave."""
+    rs = np.random.RandomState(G)
+    w = rs.standard_normal((rows, cols)).astype(np.float32)
+    cb = np.sort(rs.standard_normal(64).astype(np.float32))
+    idx = oracle.assign_nearest_np(w.ravel(), cb).reshape(rows, cols).astype(np.uint8)
+    ex = np.sort(rs.choice(rows * cols, 7, replace=False)).astype(np.int64)
+    print(f"affine rows={rows} cols={cols} G={G}", flush=True)
+    s, o = _hxq.affine_fit(torch.from_numpy(w).to(dev), torch.from_numpy(idx).to(dev), torch.from_numpy(cb).to(dev),
+                           G, torch.from_numpy(ex).to(dev))
+    so, oo = oracle.affine_fit_np(w, idx, cb, G, ex)
+    np.testing.assert_array_equal(s.cpu().numpy(), so)
+    np.testing.assert_array_equal(o.cpu().numpy(), oo)
