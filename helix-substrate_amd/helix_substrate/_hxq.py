@@ -194,25 +194,35 @@ def _check(name: str, rc: int) -> None:
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    # an int: the c_void_p argtypes take it as it is (a c_void_p object per
+    # argument and call is 0.1 us each)
+    return None if t is None else t.data_ptr()
+
+
+# torch's current stream as a raw handle: current_stream(device).cuda_stream
+# without the two objects around it (0.1 against 1.9 us a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _need_device(*ts):
-    dev = None
+    dev = index = None
     for t in ts:
         if t is None:
             continue
-        if not t.is_cuda:
+        i = t.get_device()   # -1 on the CPU
+        if i < 0 or not t.is_cuda:
             raise RuntimeError("HXQ kernels take device tensors only")
         if not t.is_contiguous():
             raise RuntimeError("HXQ kernels take contiguous tensors only")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, i
+        elif i != index:
             raise RuntimeError(f"tensors on different devices: {dev} vs {t.device}")
     return dev
 
@@ -470,16 +480,25 @@ def prefill_gemm(x, indices, codebook, group_affine, group_size, sc_grp_ptr, sc_
         raise ValueError("sc_grp_ptr must hold one pointer per (64-row group, 64-column step) "
                          "plus the end (hxq_format.sidecar_row_groups)")
     L = lib()
-    with torch.cuda.device(x.device):
-        nbytes = L.hxq_prefill_gemm_workspace_bytes(m, out_f, in_f)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes > 0 else None
-        rc = L.hxq_prefill_gemm(_ptr(x), dtype_code(x.dtype), fmt, _ptr(indices), _ptr(codebook),
-                                n_codes, _ptr(group_affine), int(group_size), _ptr(sc_grp_ptr),
-                                _ptr(sc_grp_key), _ptr(sc_grp_val), _ptr(bias), _ptr(out),
-                                dtype_code(out.dtype), m, out_f, in_f, _ptr(ws), nbytes,
-                                _stream(x))
+    if torch.cuda.current_device() != x.get_device():  # the plan asks the current device
+        with torch.cuda.device(x.device):
+            rc = _prefill_call(L, x, m, out_f, in_f, fmt, indices, codebook, n_codes, group_affine,
+                               group_size, sc_grp_ptr, sc_grp_key, sc_grp_val, bias, out)
+    else:
+        rc = _prefill_call(L, x, m, out_f, in_f, fmt, indices, codebook, n_codes, group_affine,
+                           group_size, sc_grp_ptr, sc_grp_key, sc_grp_val, bias, out)
     _check("hxq_prefill_gemm", rc)
     return out
+
+
+def _prefill_call(L, x, m, out_f, in_f, fmt, indices, codebook, n_codes, group_affine, group_size,
+                  sc_grp_ptr, sc_grp_key, sc_grp_val, bias, out):
+    nbytes = L.hxq_prefill_gemm_workspace_bytes(m, out_f, in_f)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes > 0 else None
+    return L.hxq_prefill_gemm(_ptr(x), dtype_code(x.dtype), fmt, _ptr(indices), _ptr(codebook),
+                              n_codes, _ptr(group_affine), int(group_size), _ptr(sc_grp_ptr),
+                              _ptr(sc_grp_key), _ptr(sc_grp_val), _ptr(bias), _ptr(out),
+                              dtype_code(out.dtype), m, out_f, in_f, _ptr(ws), nbytes, _stream(x))
 
 
 def gemm_noalloc(x, indices, codebook, group_affine, group_size, sc_row_ptr, sc_col, sc_val,
@@ -694,7 +713,7 @@ def gated_rmsnorm(y, gate, weight, eps, group_size=0, out_dtype=None):
     if not gate.is_cuda:
         raise RuntimeError("HXQ kernels take device tensors only")
     _need_device(y, weight, out)
-    rc = lib().hxq_gated_rmsnorm(_ptr(y), dtype_code(y.dtype), ctypes.c_void_p(gate.data_ptr()),
+    rc = lib().hxq_gated_rmsnorm(_ptr(y), dtype_code(y.dtype), gate.data_ptr(),
                                  dtype_code(gate.dtype), gate.stride(0), _ptr(weight), float(eps),
                                  rows, width, int(group_size), _ptr(out), dtype_code(out.dtype),
                                  _stream(y))

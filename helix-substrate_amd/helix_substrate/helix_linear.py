@@ -324,8 +324,8 @@ class HelixLinear(nn.Module):
         `need` (16: GEMV, 64: GEMM): the stored layout when in_features is one,
         else the padded copy and x padded with zero columns."""
         if self.in_features % need == 0:
-            return x2, self.indices
-        return pad_columns(x2, self._kin), self._kidx
+            return x2, self._buffers["indices"]
+        return pad_columns(x2, self._kin), self._buffers["_kidx"]
 
     def _pair_index_at(self, rows: torch.Tensor, pairs: torch.Tensor) -> torch.Tensor:
         """Pair index at (row, pair column), from int16 or 12-bit packed storage."""
@@ -355,7 +355,7 @@ class HelixLinear(nn.Module):
         copy, rebuilt whenever the codebook tensor, its contents version or its device
         changes (e.g. after load_state_dict or .to()).  Codebooks above 256 entries
         (int16 indices) are read as they are: those kernels take the entry count."""
-        cb = self.codebook
+        cb = self._buffers["codebook"]
         if cb.dtype == torch.float32 and cb.numel() == 256 and cb.is_contiguous():
             return cb
         if cb.numel() > 256:
@@ -418,7 +418,7 @@ class HelixLinear(nn.Module):
         """Return ``x @ W^T + bias`` in x's dtype (reference helix_linear.py:318-361)."""
         input_dtype = x.dtype
         if x.is_cuda:
-            if not self.codebook.is_cuda:
+            if not self._buffers["codebook"].is_cuda:
                 raise RuntimeError("HelixLinear buffers are on the CPU but the input is on the GPU")
             out = self._forward_hip(x)
         elif getattr(self, "_wave_enabled", False):
@@ -431,16 +431,15 @@ class HelixLinear(nn.Module):
             out = out.to(input_dtype)
         return out
 
-    def _sidecar_args(self, x2):
-        if self._sc_row_ptr is None or not self._policy_decide(x2):
-            return None, None, None
-        return self._sc_row_ptr, self._sc_col, self._sc_delta
-
     def _forward_hip(self, x: torch.Tensor) -> torch.Tensor:
+        # the buffers by their dict: nn.Module's attribute lookup is 0.3 us each,
+        # a third of a call whose kernel takes 5 us
+        b = self._buffers
         orig_shape = x.shape
-        x2 = x.reshape(-1, self.in_features)
+        K = self.in_features
+        x2 = x if x.dim() == 2 and orig_shape[1] == K else x.reshape(-1, K)
         if self.has_channel_scales:
-            x2 = x2 / self.channel_scales.unsqueeze(0)
+            x2 = x2 / b["channel_scales"].unsqueeze(0)
         if x2.dtype not in (torch.float32, torch.bfloat16, torch.float16):
             x2 = x2.float()
         x2 = x2.contiguous()
@@ -451,8 +450,9 @@ class HelixLinear(nn.Module):
         n = x2.shape[0]
         svd_on = self.has_svd and not self._cell_skip_svd
         out_dtype = torch.float32 if svd_on else x2.dtype
-        rp, col, delta = self._sidecar_args(x2)
-        out = torch.empty(n, self.out_features, dtype=out_dtype, device=x2.device)
+        sidecar = b["_sc_row_ptr"] is not None and self._policy_decide(x2)
+        out = torch.empty((n, self.out_features), dtype=out_dtype, device=x2.device)
+        fmt = self._fmt
         if n == 0:
             pass
         elif n > _GEMV_MAX_ROWS:
@@ -461,34 +461,32 @@ class HelixLinear(nn.Module):
             # fp32 ones)
             self._last_dispatch_path = "hip_gemm"
             xk, idx = self._kernel_rows(x2, 64)
-            grp = rp is not None
-            scalar8 = self._fmt == _hxq.FMT_SCALAR
-            _hxq.prefill_gemm(xk, idx, self._kcb if scalar8 else self.codebook,
-                              self._affine_t, self.group_size,
-                              self._sc_grp_ptr if grp else None,
-                              self._sc_grp_key if grp else None,
-                              self._sc_grp_val if grp else None, self.bias, out=out,
-                              fmt=self._fmt, out_features=self.out_features)
+            _hxq.prefill_gemm(xk, idx, self._kcb if fmt == _hxq.FMT_SCALAR else b["codebook"],
+                              b["_affine_t"], self.group_size,
+                              b["_sc_grp_ptr"] if sidecar else None,
+                              b["_sc_grp_key"] if sidecar else None,
+                              b["_sc_grp_val"] if sidecar else None, b["bias"], out=out,
+                              fmt=fmt, out_features=self.out_features)
         else:
             xk, idx = self._kernel_rows(x2, 16)
-            if self._fmt != _hxq.FMT_SCALAR:
-                self._last_dispatch_path = "hip_gemv_fmt"
-            else:
-                self._last_dispatch_path = "hip_gemv"
-            for r0, r1 in self._gemv_row_groups(n, xk.shape[1]):
-                if self._fmt != _hxq.FMT_SCALAR:
-                    _hxq.gemv_fmt(xk[r0:r1], self._fmt, idx, self.out_features,
-                                  codebook=self.codebook, group_scale=self.group_scale,
-                                  group_offset=self.group_offset, group_size=self.group_size,
-                                  sc_row_ptr=rp, sc_col=col, sc_delta=delta, bias=self.bias,
-                                  out=out[r0:r1])
+            rp, col, delta = ((b["_sc_row_ptr"], b["_sc_col"], b["_sc_delta"]) if sidecar
+                              else (None, None, None))
+            self._last_dispatch_path = "hip_gemv" if fmt == _hxq.FMT_SCALAR else "hip_gemv_fmt"
+            groups = self._gemv_row_groups(n, xk.shape[1])
+            for r0, r1 in groups:
+                xs, ys = (xk, out) if len(groups) == 1 else (xk[r0:r1], out[r0:r1])
+                if fmt != _hxq.FMT_SCALAR:
+                    _hxq.gemv_fmt(xs, fmt, idx, self.out_features, codebook=b["codebook"],
+                                  group_scale=b["group_scale"], group_offset=b["group_offset"],
+                                  group_size=self.group_size, sc_row_ptr=rp, sc_col=col,
+                                  sc_delta=delta, bias=b["bias"], out=ys)
                 else:
-                    _hxq.gemv(xk[r0:r1], idx, self._kcb, self.group_scale, self.group_offset,
-                              self.group_size, rp, col, delta, self.bias, out=out[r0:r1])
+                    _hxq.gemv(xs, idx, self._kcb, b["group_scale"], b["group_offset"],
+                              self.group_size, rp, col, delta, b["bias"], out=ys)
         if svd_on:
             xf = x2.float()
-            out += ((xf @ self.svd_Vt.t()) * self.svd_s.unsqueeze(0)) @ self.svd_U.t()
-        return out.reshape(*orig_shape[:-1], self.out_features)
+            out += ((xf @ b["svd_Vt"].t()) * b["svd_s"].unsqueeze(0)) @ b["svd_U"].t()
+        return out if x2 is x else out.reshape(*orig_shape[:-1], self.out_features)
 
     def _gemv_row_groups(self, n, k):
         """Row ranges of the GEMV launches for n activation rows of k columns:
