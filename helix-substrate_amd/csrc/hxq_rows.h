@@ -70,6 +70,58 @@ struct Call {
     Args a;
 };
 
+// Grouped (mixture-of-experts) launches: the rows of Y are the expert-sorted
+// assignment list, a block takes one row tile of one expert and one run of one
+// bank's subtiles.  Eight waves a block, two blocks per CU: one's table and
+// first loads pass while the other computes.
+struct Bank {
+    const uint8_t *idx;
+    const float *cb;
+    const float2 *ga;
+    const int32_t *sc_ptr;
+    const uint32_t *sc_key;
+    const float *sc_val;
+};
+
+struct Grouped {
+    Bank bank[2];            // columns [0, OUT) of Y from bank 0, [OUT, 2 OUT) from bank 1
+    const int32_t *rows;     // X row of each sorted position (null: the position)
+    const int32_t *seg;      // expert e owns positions [seg[e], seg[e + 1])
+    int32_t n_exp, n_banks, x_rows, runs;   // runs: blocks per bank and row tile
+    int64_t idx_es, ga_es, scp_es;          // per-expert strides (codebooks: 256)
+};
+
+// Row tile rt (of bm rows, counted over all experts): its expert, first position
+// and the segment's end; false past the last one.  Every wave alike, by wave
+// scans.
+__device__ __forceinline__ bool row_tile(const Grouped &g, int bm, int rt, int &e, int &row0, int &rend) {
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int c0 = 0; c0 < g.n_exp; c0 += 64) {
+        const int ee = c0 + lane;
+        const int a = ee < g.n_exp ? g.seg[ee] : 0;
+        const int b = ee < g.n_exp ? g.seg[ee + 1] : 0;
+        const int nt = (b - a + bm - 1) / bm;
+        int inc = nt;
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x111, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x112, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x114, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x118, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);
+        const int tot = __builtin_amdgcn_readlane(inc, 63);
+        if (rt < base + tot) {
+            const int l = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(base + inc > rt)));
+            e = c0 + l;
+            row0 = __builtin_amdgcn_readlane(a, l) + (rt - base - __builtin_amdgcn_readlane(inc - nt, l)) * bm;
+            rend = __builtin_amdgcn_readlane(b, l);
+            return true;
+        }
+        base += tot;
+    }
+    return false;
+}
+
 // index bytes per 16 weights
 __host__ __device__ constexpr int fmt_b16(int f) {
     return f == HXQ_FMT_SCALAR_U16 ? 32 : (f == HXQ_FMT_VQ2_P12 || f == HXQ_FMT_AF6) ? 12 : 16;
@@ -91,11 +143,12 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 // steps per iteration; XT: 0 fp16, 1 bf16, 2 fp32; W: waves per block.
 // The arguments that the first loads need come first, as scalars: they are
 // preloaded into SGPRs, so no argument fetch precedes the stream.
-template <int MT, int NS, int SP, int XT, bool AFF, int FMT, int W>
-__global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, const void *a_x, const float *a_cb,
+template <int MT, int NS, int SP, int XT, bool AFF, int FMT, int W, bool GRP = false>
+__global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t *a_idx, const void *a_x, const float *a_cb,
                                                       const float2 *a_ga, const int32_t M, const int32_t OUT,
                                                       const int32_t K, const int32_t ngroups,
-                                                      const uint32_t gmul, const Args g) {
+                                                      const uint32_t gmul, const Args g,
+                                                      const typename std::conditional<GRP, Grouped, int>::type grp) {
     constexpr bool F32 = XT == 2;
     constexpr int XB = F32 ? 4 : 2;
     constexpr int XCH = kStep * XB / 16;      // 16-byte chunks per X row and step
@@ -118,8 +171,37 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, hq = lane >> 4;
-    const int n0 = blockIdx.x * (NS * kSub);
-    const int m0 = blockIdx.y * (MT * kSub);  // first row of X and Y
+    int n0 = blockIdx.x * (NS * kSub);
+    int m0 = blockIdx.y * (MT * kSub);  // first row of X and Y
+    int mend = M, ybase = 0, ywidth = OUT;
+    int64_t xrows = M;
+    const int32_t *sc_ptr = g.sc_ptr;
+    const uint32_t *sc_key = g.sc_key;
+    const float *sc_val = g.sc_val;
+    int nnz = 0;
+    if constexpr (GRP) {
+        int e, w = blockIdx.x % (grp.runs * grp.n_banks);
+        if (!row_tile(grp, MT * kSub, blockIdx.x / (grp.runs * grp.n_banks), e, m0, mend)) return;  // block-uniform
+        const Bank &b = grp.bank[w >= grp.runs];
+        if (w >= grp.runs) {
+            w -= grp.runs;
+            ybase = OUT;
+        }
+        n0 = w * (NS * kSub);
+        ywidth = OUT * grp.n_banks;
+        xrows = grp.x_rows;
+        a_idx = b.idx + e * grp.idx_es;
+        a_cb = b.cb + e * 256;
+        a_ga = b.ga + e * grp.ga_es;
+        sc_key = b.sc_key;
+        sc_val = b.sc_val;
+        if (b.sc_ptr) {   // the lists of all experts are one: its length after the last expert's last step
+            nnz = kload(b.sc_ptr[grp.n_exp * grp.scp_es - 1]);
+            sc_ptr = b.sc_ptr + e * grp.scp_es;
+        } else {
+            sc_ptr = nullptr;
+        }
+    }
     const int nst = K / kStep;
     char *sx = smem + kTbl + wave * kX;
 
@@ -131,7 +213,7 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
     // K = 18944, 16 rows, of which X alone 16).  Indices change lanes by
     // ds_bpermute, X through the wave's LDS tile.
     const int64_t row_bytes = (int64_t)K / 16 * B16;
-    const int64_t x_bytes = (int64_t)M * K * XB, q_bytes = (int64_t)OUT * row_bytes;
+    const int64_t x_bytes = xrows * K * XB, q_bytes = (int64_t)OUT * row_bytes;
     const int64_t a_bytes = (int64_t)ngroups * OUT * 8;
     uint32_t x_off[MT][NX], q_off[NS];
 #pragma unroll
@@ -139,7 +221,9 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
 #pragma unroll
         for (int q = 0; q < NX; ++q) {
             const int m = m0 + 16 * i + lane / XCH + (64 / XCH) * q;
-            x_off[i][q] = m < M ? static_cast<uint32_t>(m * K * XB + (lane % XCH) * 16) : kOob;
+            int row = m;
+            if constexpr (GRP) row = m < mend && grp.rows ? grp.rows[m] : m;
+            x_off[i][q] = m < mend ? static_cast<uint32_t>(row * K * XB + (lane % XCH) * 16) : kOob;
         }
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
@@ -193,7 +277,7 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
     };
     // sidecar: lanes 0-31 the run's first 64-row group, 32-63 the next one;
     // the pointers of an iteration two ahead, its entries one ahead
-    const bool has_sc = g.sc_ptr != nullptr;
+    const bool has_sc = sc_ptr != nullptr;
     const int ngrp = (OUT + 63) >> 6;
     const int half = lane >> 5;
     const uint32_t l32 = lane & 31u;
@@ -201,15 +285,15 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
     const int rbase = sgrp * 64 - n0;         // row of the run of the group's first row
     const uint32_t p_off = sgrp < ngrp ? static_cast<uint32_t>(sgrp * nst) * 4u : kOob;
     const int64_t p_bytes = has_sc ? int64_t{4} * (ngrp * nst + 1) : 0;
-    const int nnz = has_sc ? kload(g.sc_ptr[ngrp * nst]) : 0;
-    const __amdgpu_buffer_rsrc_t kr = make_rsrc(g.sc_key, int64_t{4} * nnz);
-    const __amdgpu_buffer_rsrc_t vr = make_rsrc(g.sc_val, int64_t{4} * nnz);
+    if constexpr (!GRP) nnz = has_sc ? kload(sc_ptr[ngrp * nst]) : 0;
+    const __amdgpu_buffer_rsrc_t kr = make_rsrc(sc_key, int64_t{4} * nnz);
+    const __amdgpu_buffer_rsrc_t vr = make_rsrc(sc_val, int64_t{4} * nnz);
     uint32_t pf, pl;          // first entry and end of an iteration's steps
     uint32_t se, sn;          // this lane's list index, the group's entry count
     uint32_t sk;
     float sv;
     auto load_ptr = [&](int t) {
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(g.sc_ptr, t < nst ? p_bytes : 0);
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(sc_ptr, t < nst ? p_bytes : 0);
         const int so = t < nst ? t * 4 : 0;
         pf = __builtin_amdgcn_raw_buffer_load_b32(r, p_off, so, 0);
         pl = __builtin_amdgcn_raw_buffer_load_b32(r, p_off + 4u * min(SP, max(nst - t, 0)), so, 0);
@@ -392,7 +476,7 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
                     for (uint32_t e = e0 + 32; __ballot(e < en) != 0; e += 32) {
                         const bool in = e < en;
                         uint32_t w2, c2, v2;
-                        place(in ? g.sc_key[e] : 0u, in ? g.sc_val[e] : 0.f, in, t, w2, c2, v2);
+                        place(in ? sc_key[e] : 0u, in ? sc_val[e] : 0.f, in, t, w2, c2, v2);
                         apply(__ballot(w2 == j + 8u * s), c2, v2, b);
                     }
                 }
@@ -440,12 +524,12 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
         const int l = it & 63, i = (it >> 6) % MT, j = (it >> 6) / MT;
         const int m = m0 + 16 * i + (l & 15);
         const int n = n0 + kSub * j + 4 * (l >> 4);  // C layout: rows 4 (lane / 16) + r
-        if (m >= M || n >= OUT) continue;
+        if (m >= mend || n >= OUT) continue;
         const int nv = min(4, OUT - n);
         float v[4] = {s[0], s[1], s[2], s[3]};
         if (g.bias)
             for (int r = 0; r < nv; ++r) v[r] += g.bias[n + r];
-        const int64_t o = (int64_t)m * OUT + n;
+        const int64_t o = (int64_t)m * ywidth + ybase + n;
         if (g.y_dtype == HXQ_F32) {
             float *y = static_cast<float *>(g.y) + o;
             if (g.vec_out && nv == 4) *reinterpret_cast<float4 *>(y) = make_float4(v[0], v[1], v[2], v[3]);
@@ -466,8 +550,11 @@ __global__ __launch_bounds__(W * 64) void rows_kernel(const uint8_t *a_idx, cons
 }
 
 constexpr int kMaxRows = 64, kMaxRowsF32 = 32;
+constexpr int kGroupedSubs = 5;  // subtiles per block of a grouped launch (16-row tiles)
 
 // Launches the kernel for XT with mt row tiles and ns subtiles per block.
+template <int XT>
+int launch_grouped(const Call &c, const Grouped &g, bool aff, int blocks, hipStream_t stream);
 template <int XT>
 int launch_rows(const Call &c, int format, bool aff, const Plan &p, hipStream_t stream);
 

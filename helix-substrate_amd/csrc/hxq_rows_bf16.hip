@@ -3,5 +3,6 @@
 namespace hxq {
 namespace rw {
 template int launch_rows<1>(const Call &, int, bool, const Plan &, hipStream_t);
+template int launch_grouped<1>(const Call &, const Grouped &, bool, int, hipStream_t);
 }  // namespace rw
 }  // namespace hxq

@@ -13,7 +13,7 @@ static int launch_fmt(const Call &c, int format, bool aff, const Plan &p, hipStr
     const dim3 grid(p.bx, p.by), block(W * 64);
 #define HXQ_RW(AF_, F_) \
     hipLaunchKernelGGL((rows_kernel<MT, NS, SP, XT, AF_, F_, W>), grid, block, 0, stream, c.idx, c.x, c.cb, \
-                       c.ga, c.M, c.OUT, c.K, c.ngroups, c.gmul, c.a)
+                       c.ga, c.M, c.OUT, c.K, c.ngroups, c.gmul, c.a, 0)
     switch (format) {
         case HXQ_FMT_SCALAR:
             if (aff) HXQ_RW(true, HXQ_FMT_SCALAR); else HXQ_RW(false, HXQ_FMT_SCALAR);
@@ -57,6 +57,18 @@ int launch_rows(const Call &c, int format, bool aff, const Plan &p, hipStream_t 
     }
 #undef HXQ_RWS
     HXQ_REQUIRE(false, "no such few-row plan");
+}
+
+// Two blocks per CU: 80 KB of LDS and 128 registers each.
+template <int XT>
+int launch_grouped(const Call &c, const Grouped &g, bool aff, int blocks, hipStream_t stream) {
+#define HXQ_RWG(AF_)                                                                                          \
+    hipLaunchKernelGGL((rows_kernel<1, kGroupedSubs, 1, XT, AF_, HXQ_FMT_SCALAR, 8, true>), dim3(blocks),      \
+                       dim3(512), 0, stream, c.idx, c.x, c.cb, c.ga, c.M, c.OUT, c.K, c.ngroups, c.gmul, c.a, g)
+    if (aff) HXQ_RWG(true); else HXQ_RWG(false);
+#undef HXQ_RWG
+    HXQ_LAUNCH_CHECK();
+    return HXQ_OK;
 }
 
 }  // namespace rw

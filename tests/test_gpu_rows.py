@@ -71,3 +71,31 @@ def test_rows_formats(dev, fmt, m, out, inp, xdt):
 def test_rows_dense_sidecar(dev, m, out, inp, xdt):
     """5 % of the weights: some 200 entries per row group and step."""
     _check(dev, _hxq.FMT_SCALAR, m, out, inp, 128, xdt, density=0.05)
+
+
+@pytest.mark.parametrize("counts", [(1,), (0, 1, 0, 16), (17, 0, 3, 33), (0, 0, 5), (2, 2, 2, 2, 2, 2, 2)])
+@pytest.mark.parametrize("out,inp", [(64, 64), (336, 576), (1024, 2048)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_rows_grouped(dev, counts, out, inp, xdt):
+    """Experts of few, no and just over 16 rows; runs of five subtiles that end inside a block."""
+    from helix_substrate import synth
+    from helix_substrate.moe import bank_to, stack_bank
+    E, n = len(counts), sum(counts)
+    Ls = [synth.make_layer_np(out, inp, seed=e, group_size=64, density=0.01) for e in range(E)]
+    bank = bank_to(stack_bank([synth.to_torch(L) for L in Ls]), dev)
+    bank["group_size"] = 64
+    g = torch.Generator().manual_seed(n)
+    rows = torch.randint(0, 9, (n,), generator=g).to(torch.int32)
+    x = torch.randn(9, inp, generator=g).to(xdt)
+    off = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32)
+    print(f"rows grouped counts={counts} out={out} in={inp} x={xdt}", flush=True)
+    y = _hxq.moe_grouped_gemm(x.to(dev), rows.to(dev), off.to(dev), bank, n).cpu().numpy()
+    for e, L in enumerate(Ls):
+        lo, hi = int(off[e]), int(off[e + 1])
+        if lo == hi:
+            continue
+        W = oracle.reconstruct(L["indices"], L["codebook"], L["group_scale"], L["group_offset"], 64,
+                               L["sidecar_positions"], L["sidecar_values"], fma=True)
+        W16 = torch.from_numpy(W).to(xdt).float().numpy()
+        ref = oracle.linear_np(x[rows[lo:hi].long()].float().numpy(), W16)
+        assert _maxrel(y[lo:hi], ref) <= 2e-5, e   # operands equal: order of fp32 sums
