@@ -32,6 +32,8 @@ struct ConvArgs {
     float dt_min, dt_max;
     int32_t batch, seqlen, proj_width, xbc_off, dt_off, d_inner, gn, heads, width;
     int32_t proj_dt, out_dt;
+    int32_t steps;           // time steps per block of the vector kernel
+    int32_t bias_vec, state_vec;  // bias, conv_state are 16-byte aligned
 };
 
 __device__ __forceinline__ float ld16or32(const void *p, int64_t i, int dt) {
@@ -46,7 +48,32 @@ __device__ __forceinline__ void st16or32(void *p, int64_t i, int dt, float v) {
     else static_cast<uint16_t *>(p)[i] = f32_to_f16(v);
 }
 
-__device__ __forceinline__ float silu(float v) { return v / (1.f + expf(-v)); }
+// v / (1 + exp(-v)) to within an ulp or two in 14 instructions (the library
+// exponential and an IEEE division take 30, and bounded the convolution and
+// the gated norm: 110 us for 71M values): exp2 of -v log2(e) in two parts, the
+// hardware reciprocal with one Newton step.  -v is held to where the
+// exponential is finite; below -86 (sums over 2e37, whose reciprocal is
+// denormal) the plain reciprocal gives the limit -0.
+__device__ __forceinline__ float silu(float v) {
+    const float w = -fminf(fmaxf(v, -88.7f), 100.f);
+    const float p = w * 1.44269502f;
+    const float lo = fmaf(w, 1.92596299e-8f, fmaf(w, 1.44269502f, -p));
+    float e = __builtin_amdgcn_exp2f(p);
+    e = fmaf(e, lo * 0.693147182f, e);
+    const float d = 1.f + e;
+    const float r = __builtin_amdgcn_rcpf(d);
+    return v * (d < 2e37f ? fmaf(fmaf(-d, r, 1.f), r, r) : r);
+}
+
+// Two fp32 values rounded to nearest even in one conversion.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <bool BF16>
+__device__ __forceinline__ uint32_t pack16(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
+}
 
 // torch.nn.functional.softplus (beta 1, threshold 20)
 __device__ __forceinline__ float softplus(float v) { return v > 20.f ? v : log1pf(expf(v)); }
@@ -131,69 +158,108 @@ __global__ __launch_bounds__(256) void conv_split_kernel(const ConvArgs a) {
 // offsets multiples of 8): a thread owns 8 consecutive channels, reads each
 // time step's 8 inputs as one 16-byte load and writes the 8 outputs as one
 // 16-byte store; the W-1 previous inputs of its channels stay in registers
-// (W <= 4).  dt channels keep the scalar kernel (a second launch).
+// (W <= 4).  The grid's last column of blocks does the dt channels.  Bound by
+// memory latency and the SiLU's arithmetic: 8 x 2048 tokens of 4352 channels
+// 152 to 97 us with the short silu() above, the taps by way of LDS, the next
+// round's rows requested ahead and the dt channels in the same launch.
 template <int W, bool BF16>
 __global__ __launch_bounds__(256) void conv_split_vec_kernel(const ConvArgs a) {
     const int conv_dim = a.d_inner + 2 * a.gn;
+    const int t0 = blockIdx.y * a.steps;
+    const int b = blockIdx.z;
+    const int t1 = min(t0 + a.steps, a.seqlen);
+    const int64_t row0 = (int64_t)b * a.seqlen;
+    if (blockIdx.x == gridDim.x - 1) {
+        for (int i = threadIdx.x; i < (t1 - t0) * a.heads; i += 256) {
+            const int h = i % a.heads;
+            const int64_t row = row0 + t0 + i / a.heads;
+            a.dt[row * a.heads + h] = dt_transform(ld16or32(a.proj, row * a.proj_width + a.dt_off + h, a.proj_dt), a, h);
+        }
+        return;
+    }
     const int cg = blockIdx.x * 256 + threadIdx.x;  // channel group: channels 8 cg .. 8 cg + 7
     const int c0 = 8 * cg;
-    if (c0 >= conv_dim) return;
-    const int t0 = blockIdx.y * kConvT;
-    const int b = blockIdx.z;
-    const int t1 = min(t0 + kConvT, a.seqlen);
-    const int64_t row0 = (int64_t)b * a.seqlen;
+    const bool live = c0 < conv_dim;
     float w[8][W], bias[8], win[W > 1 ? W - 1 : 1][8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-#pragma unroll
-        for (int k = 0; k < W; ++k) w[j][k] = a.w[(int64_t)(c0 + j) * W + k];
-        bias[j] = a.bias ? a.bias[c0 + j] : 0.f;
-    }
-    const uint16_t *proj = static_cast<const uint16_t *>(a.proj);
-    auto load8 = [&](int64_t t, float (&v)[8]) {
-        const u32x4 q = *reinterpret_cast<const u32x4 *>(proj + (row0 + t) * a.proj_width + a.xbc_off + c0);
+    // the window's rows and the first round's, requested before the taps
+    const uint16_t *proj = static_cast<const uint16_t *>(a.proj) + (live ? c0 : 0) + a.xbc_off;
+    auto row = [&](int t) { return *reinterpret_cast<const u32x4 *>(proj + (row0 + t) * a.proj_width); };
+    auto widen = [&](const u32x4 &q, float (&v)[8]) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const uint16_t h = static_cast<uint16_t>(q[j >> 1] >> (16 * (j & 1)));
             v[j] = BF16 ? bf16_to_f32(h) : f16_to_f32(h);
         }
     };
+    u32x4 qw[W > 1 ? W - 1 : 1], qin[2][kConvTB];
     // window slot k holds input t - (W - 1) + k (zero before t = 0)
 #pragma unroll
     for (int k = 0; k < W - 1; ++k) {
         const int tt = t0 - (W - 1) + k;
-        if (tt >= 0) load8(tt, win[k]);
-        else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) win[k][j] = 0.f;
-        }
+        qw[k] = row(max(tt, 0));
+        if (tt < 0) qw[k] = u32x4{0u, 0u, 0u, 0u};
     }
+    auto request = [&](int tb, u32x4 (&q)[kConvTB]) {
+#pragma unroll
+        for (int i = 0; i < kConvTB; ++i) q[i] = row(min(tb + i, t1 - 1));  // past t1: a repeat, unused
+    };
+    request(t0, qin[0]);
+    if constexpr (W == 4) {
+        // the block's taps by way of LDS: a thread's own eight channels are 128
+        // bytes apart from its neighbour's, a line per lane and load (2.5 us of
+        // a CU per block, as long as three rounds of its steps).  A channel's
+        // 16 bytes sit at c ^ (c / 8) % 8: two lanes a bank group, not sixteen.
+        __shared__ float4 sw[2048];
+        const int cb = blockIdx.x * 2048, nc = min(2048, conv_dim - cb);
+        const float4 *gw = reinterpret_cast<const float4 *>(a.w) + cb;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = threadIdx.x + 256 * i;
+            if (c < nc) sw[c ^ ((c >> 3) & 7)] = gw[c];
+        }
+        __syncthreads();
+        if (!live) return;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int c = 8 * threadIdx.x + j;
+            const float4 q = sw[c ^ ((c >> 3) & 7)];
+            w[j][0] = q.x;
+            w[j][1] = q.y;
+            w[j][2] = q.z;
+            w[j][3] = q.w;
+        }
+    } else {
+        if (!live) return;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int k = 0; k < W; ++k) w[j][k] = a.w[(int64_t)(c0 + j) * W + k];
+    }
+    if (a.bias && a.bias_vec) {
+        const float4 b0 = reinterpret_cast<const float4 *>(a.bias + c0)[0], b1 = reinterpret_cast<const float4 *>(a.bias + c0)[1];
+        bias[0] = b0.x; bias[1] = b0.y; bias[2] = b0.z; bias[3] = b0.w;
+        bias[4] = b1.x; bias[5] = b1.y; bias[6] = b1.z; bias[7] = b1.w;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bias[j] = a.bias ? a.bias[c0 + j] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < W - 1; ++k) widen(qw[k], win[k]);
     // destination: x, B or C (a group of 8 never straddles them)
     uint16_t *dst;
     int64_t dstride, doff;
     if (c0 < a.d_inner) { dst = static_cast<uint16_t *>(a.x); dstride = a.d_inner; doff = c0; }
     else if (c0 < a.d_inner + a.gn) { dst = static_cast<uint16_t *>(a.B); dstride = a.gn; doff = c0 - a.d_inner; }
     else { dst = static_cast<uint16_t *>(a.C); dstride = a.gn; doff = c0 - a.d_inner - a.gn; }
-    const bool obf = a.out_dt == HXQ_BF16;
-    // kConvTB time steps per round: their inputs are all requested before the
-    // first is used (one memory round trip per round, not per step)
-    for (int tb = t0; tb < t1; tb += kConvTB) {
-        u32x4 qin[kConvTB];
-#pragma unroll
-        for (int i = 0; i < kConvTB; ++i) {
-            const int t = min(tb + i, t1 - 1);  // past t1: a repeat of a loaded row, unused
-            qin[i] = *reinterpret_cast<const u32x4 *>(proj + (row0 + t) * a.proj_width + a.xbc_off + c0);
-        }
+    // kConvTB time steps per round, the next round's inputs requested before
+    // this one is computed
+    auto round = [&](int tb, const u32x4 (&q)[kConvTB]) {
 #pragma unroll
         for (int i = 0; i < kConvTB; ++i) {
             const int t = tb + i;
             if (t >= t1) break;
             float cur[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint16_t h = static_cast<uint16_t>(qin[i][j >> 1] >> (16 * (j & 1)));
-                cur[j] = BF16 ? bf16_to_f32(h) : f16_to_f32(h);
-            }
+            widen(q[i], cur);
             uint32_t o[4];
 #pragma unroll
             for (int j2 = 0; j2 < 4; ++j2) {
@@ -207,8 +273,7 @@ __global__ __launch_bounds__(256) void conv_split_vec_kernel(const ConvArgs a) {
                     acc = fmaf(w[j][W - 1], cur[j], acc);
                     r[e] = silu(acc);
                 }
-                o[j2] = obf ? (uint32_t(f32_to_bf16(r[0])) | (uint32_t(f32_to_bf16(r[1])) << 16))
-                            : (uint32_t(f32_to_f16(r[0])) | (uint32_t(f32_to_f16(r[1])) << 16));
+                o[j2] = pack16<BF16>(r[0], r[1]);   // (the outputs have proj's type)
             }
             *reinterpret_cast<u32x4 *>(dst + (row0 + t) * dstride + doff) = u32x4{o[0], o[1], o[2], o[3]};
 #pragma unroll
@@ -220,32 +285,38 @@ __global__ __launch_bounds__(256) void conv_split_vec_kernel(const ConvArgs a) {
                 for (int j = 0; j < 8; ++j) win[W - 2][j] = cur[j];
             }
         }
+    };
+    for (int tb = t0; tb < t1; tb += 2 * kConvTB) {
+        request(tb + kConvTB, qin[1]);
+        round(tb, qin[0]);
+        if (tb + kConvTB >= t1) break;
+        request(tb + 2 * kConvTB, qin[0]);
+        round(tb + kConvTB, qin[1]);
     }
     // conv_state after the last step: the last W raw inputs (zero before t=0)
     if (a.conv_state && t1 == a.seqlen) {
+        u32x4 q[W];
+        float v[W][8];
+#pragma unroll
+        for (int k = 0; k < W; ++k) q[k] = row(max(a.seqlen - W + k, 0));
 #pragma unroll
         for (int k = 0; k < W; ++k) {
-            const int tt = a.seqlen - W + k;
-            float v[8];
-            if (tt >= 0) load8(tt, v);
-            else {
+            if (a.seqlen - W + k < 0) q[k] = u32x4{0u, 0u, 0u, 0u};
+            widen(q[k], v[k]);
+        }
+        float *cs = a.conv_state + ((int64_t)b * conv_dim + c0) * W;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = 0.f;
+        for (int j = 0; j < 8; ++j) {
+            if constexpr (W == 4) {
+                if (a.state_vec) {
+                    reinterpret_cast<float4 *>(cs)[j] = make_float4(v[0][j], v[1][j], v[2][j], v[3][j]);
+                    continue;
+                }
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) a.conv_state[((int64_t)b * conv_dim + c0 + j) * W + k] = v[j];
+            for (int k = 0; k < W; ++k) cs[j * W + k] = v[k][j];
         }
     }
-}
-
-// dt channels only (the vector conv kernel covers x/B/C)
-__global__ __launch_bounds__(256) void dt_kernel(const ConvArgs a) {
-    const int64_t i = blockIdx.x * 256ll + threadIdx.x;  // (row, head)
-    const int64_t n = (int64_t)a.batch * a.seqlen * a.heads;
-    if (i >= n) return;
-    const int64_t row = i / a.heads;
-    const int h = static_cast<int>(i % a.heads);
-    a.dt[i] = dt_transform(ld16or32(a.proj, row * a.proj_width + a.dt_off + h, a.proj_dt), a, h);
 }
 
 // Decode: one token per batch row; conv_state [b, conv_dim, W] rolls left and
@@ -483,10 +554,21 @@ extern "C" int hxq_mamba2_conv_split(const void *proj, int32_t proj_dtype, const
                      a.proj_width % 8 == 0 && a.xbc_off % 8 == 0 && a.d_inner % 8 == 0 &&
                      a.gn % 8 == 0 &&
                      ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(x) |
-                       reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) & 15u) == 0;
+                       reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) & 15u) == 0 &&
+                     (width != 4 || (reinterpret_cast<uintptr_t>(conv_w) & 15u) == 0);
+    a.bias_vec = (reinterpret_cast<uintptr_t>(conv_b) & 15u) == 0;
+    a.state_vec = (reinterpret_cast<uintptr_t>(conv_state) & 15u) == 0;
     if (vec) {
         const int groups = (a.d_inner + 2 * a.gn) / 8;
-        const dim3 grid((groups + 255) / 256, (a.seqlen + kConvT - 1) / kConvT, a.batch);
+        // 16 steps per block (taps and window read once in 16) while that gives
+        // every CU a block, fewer below: us at 16 / 8 / 4 steps, 4352 channels:
+        // 8 x 2048 tokens 97 / 105 / 125, 2 x 1000 18.9 / 22.0 / 22.4, 512
+        // 14.4 / 11.5 / 11.7, 64 12.2 / 9.1 / 7.6
+        const int gx = (groups + 255) / 256;
+        const int64_t blocks = static_cast<int64_t>(gx) * a.batch * ((a.seqlen + kConvT - 1) / kConvT);
+        const int cus = device_cu_count();
+        a.steps = blocks >= cus ? kConvT : 4 * blocks >= cus ? kConvT / 2 : kConvTB;
+        const dim3 grid(gx + 1, (a.seqlen + a.steps - 1) / a.steps, a.batch);
         const bool bf = proj_dtype == HXQ_BF16;
         switch (width) {
             case 1: if (bf) hipLaunchKernelGGL((conv_split_vec_kernel<1, true>), grid, dim3(256), 0, stream, a);
@@ -502,9 +584,6 @@ extern "C" int hxq_mamba2_conv_split(const void *proj, int32_t proj_dtype, const
                      else hipLaunchKernelGGL((conv_split_vec_kernel<4, false>), grid, dim3(256), 0, stream, a);
                      break;
         }
-        HXQ_LAUNCH_CHECK();
-        const int64_t n = (int64_t)a.batch * a.seqlen * a.heads;
-        hipLaunchKernelGGL(dt_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, stream, a);
         HXQ_LAUNCH_CHECK();
         return HXQ_OK;
     }

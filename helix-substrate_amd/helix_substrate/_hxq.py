@@ -526,17 +526,23 @@ def gemm_noalloc(x, indices, codebook, group_affine, group_size, sc_row_ptr, sc_
 
 
 def ssm_chunk_scan(x, dt, A, B, C, D=None, h0=None, chunk=256, out_dtype=torch.float32,
-                   want_final=True):
+                   want_final=True, final=None):
     """Selective scan on the GPU.  x [b, L, H, P], dt [b, L, H], A [H], B/C [b, L, G, N],
-    D [H] (or [H, 1]), h0 [b, H, P, N] fp32 or None.  Returns (y, h_final)."""
+    D [H] (or [H, 1]), h0 [b, H, P, N] fp32 or None.  Returns (y, h_final); final: an
+    fp32 [b, H, P, N] tensor to take h_final (may not overlap h0)."""
     batch, seqlen, heads, head_dim = x.shape
     ngroups, state = B.shape[2], B.shape[3]
     A = A.float().contiguous()
     D = None if D is None else D.float().reshape(-1).contiguous()
     h0 = None if h0 is None else h0.float().contiguous()
     y = torch.empty(batch, seqlen, heads, head_dim, dtype=out_dtype, device=x.device)
-    hf = torch.empty(batch, heads, head_dim, state, dtype=torch.float32, device=x.device) \
-        if want_final else None
+    hf = final
+    if hf is not None:
+        _need_f32(final=hf)
+        if tuple(hf.shape) != (batch, heads, head_dim, state):
+            raise ValueError("final must be [batch, heads, head_dim, state]")
+    elif want_final:
+        hf = torch.empty(batch, heads, head_dim, state, dtype=torch.float32, device=x.device)
     L = lib()
     nbytes = L.hxq_ssm_scan_workspace_bytes(batch, seqlen, heads, head_dim, state, chunk)
     if nbytes < 0:

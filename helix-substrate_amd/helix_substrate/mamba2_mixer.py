@@ -97,10 +97,16 @@ class HelixMamba2Mixer(nn.Module):
             self.ssm_state_size, self.num_heads,
             conv_state=None if state is None else state[0])
         A = -torch.exp(self.A_log)
-        y, h = _hxq.ssm_chunk_scan(x, dt, A, B, C, self.D, None, chunk=self.chunk_size,
-                                   out_dtype=torch.float32, want_final=state is not None)
-        if state is not None:
-            state[1].copy_(h)
+        # the final state straight into the caller's (a copy of it otherwise)
+        h = None if state is None else state[1]
+        direct = (h is not None and h.is_cuda and h.device == x.device and h.is_contiguous()
+                  and h.dtype == torch.float32 and h.data_ptr() % 16 == 0 and tuple(h.shape) ==
+                  (b, self.num_heads, self.head_dim, self.ssm_state_size))
+        y, hf = _hxq.ssm_chunk_scan(x, dt, A, B, C, self.D, None, chunk=self.chunk_size,
+                                    out_dtype=torch.float32, want_final=h is not None,
+                                    final=h if direct else None)
+        if h is not None and not direct:
+            h.copy_(hf)
         gate, _, _ = self._split(proj.view(b * L, -1))
         z = _hxq.gated_rmsnorm(y.view(b * L, -1), gate, self.norm_weight, self.variance_epsilon,
                                group_size=self.norm_group_size, out_dtype=dtype)
