@@ -450,6 +450,10 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
         load_ptr(tn + W * SP);
 #pragma unroll
         for (int s = 0; s < SP; ++s) {
+            // a step past the last would add codebook entry 0 times zero: NaN where
+            // that entry is infinite and no weight uses it (the exit: at most 1 %, 16 x
+            // 3584 x 18944 30.7 / 30.9 us, 64 x 3584 x 18944 52.2 / 52.1)
+            if (SP > 1 && t + s >= nst) break;
             // X through the wave's tile into operand layout (LDS serves a wave in order)
             u32x4 xo[MT][XCH / 4];
 #pragma unroll

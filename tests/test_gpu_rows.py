@@ -73,6 +73,24 @@ def test_rows_dense_sidecar(dev, m, out, inp, xdt):
     _check(dev, _hxq.FMT_SCALAR, m, out, inp, 128, xdt, density=0.05)
 
 
+@pytest.mark.parametrize("m,out,inp", [(16, 48, 192), (16, 48, 64 * 67), (40, 48, 192)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+def test_rows_infinite_unused_entry(dev, m, out, inp, xdt):
+    """Step counts that are no multiple of a wave's steps per iteration, with an infinite
+    codebook entry 0 that no index uses: the result is the one with that entry finite."""
+    g = torch.Generator().manual_seed(inp)
+    idx = torch.randint(1, 256, (out, inp), generator=g, dtype=torch.uint8).to(dev)
+    cb = torch.randn(256, generator=g)
+    x = torch.randn(m, inp, generator=g).to(xdt).to(dev)
+    print(f"rows inf entry m={m} out={out} in={inp} x={xdt}", flush=True)
+    ys = []
+    for v in (0.0, float("inf")):
+        cb[0] = v
+        ys.append(_hxq.prefill_gemm(x, idx, cb.to(dev), None, 128, None, None, None, None,
+                                    out_dtype=torch.float32))
+    assert torch.isfinite(ys[0]).all() and torch.equal(ys[0], ys[1])
+
+
 @pytest.mark.parametrize("counts", [(1,), (0, 1, 0, 16), (17, 0, 3, 33), (0, 0, 5), (2, 2, 2, 2, 2, 2, 2)])
 @pytest.mark.parametrize("out,inp", [(64, 64), (336, 576), (1024, 2048)])
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
