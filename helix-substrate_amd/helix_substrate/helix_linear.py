@@ -324,8 +324,8 @@ class HelixLinear(nn.Module):
         `need` (16: GEMV, 64: GEMM): the stored layout when in_features is one,
         else the padded copy and x padded with zero columns."""
         if self.in_features % need == 0:
-            return x2, self._buffers["indices"]
-        return pad_columns(x2, self._kin), self._buffers["_kidx"]
+            return x2, self._tensors()["indices"]
+        return pad_columns(x2, self._kin), self._tensors()["_kidx"]
 
     def _pair_index_at(self, rows: torch.Tensor, pairs: torch.Tensor) -> torch.Tensor:
         """Pair index at (row, pair column), from int16 or 12-bit packed storage."""
@@ -355,7 +355,7 @@ class HelixLinear(nn.Module):
         copy, rebuilt whenever the codebook tensor, its contents version or its device
         changes (e.g. after load_state_dict or .to()).  Codebooks above 256 entries
         (int16 indices) are read as they are: those kernels take the entry count."""
-        cb = self._buffers["codebook"]
+        cb = self._tensors()["codebook"]
         if cb.dtype == torch.float32 and cb.numel() == 256 and cb.is_contiguous():
             return cb
         if cb.numel() > 256:
@@ -418,7 +418,7 @@ class HelixLinear(nn.Module):
         """Return ``x @ W^T + bias`` in x's dtype (reference helix_linear.py:318-361)."""
         input_dtype = x.dtype
         if x.is_cuda:
-            if not self._buffers["codebook"].is_cuda:
+            if not self._tensors()["codebook"].is_cuda:
                 raise RuntimeError("HelixLinear buffers are on the CPU but the input is on the GPU")
             out = self._forward_hip(x)
         elif getattr(self, "_wave_enabled", False):
@@ -431,10 +431,16 @@ class HelixLinear(nn.Module):
             out = out.to(input_dtype)
         return out
 
+    def _tensors(self) -> dict:
+        """The tensors by name: the buffers' dict, with whatever a caller has assigned as a
+        Parameter (nn.Module moves that name out of the buffers; `weight` is one always)."""
+        p = self._parameters
+        return self._buffers if len(p) <= 1 else {**self._buffers, **p}
+
     def _forward_hip(self, x: torch.Tensor) -> torch.Tensor:
         # the buffers by their dict: nn.Module's attribute lookup is 0.3 us each,
         # a third of a call whose kernel takes 5 us
-        b = self._buffers
+        b = self._tensors()
         orig_shape = x.shape
         K = self.in_features
         x2 = x if x.dim() == 2 and orig_shape[1] == K else x.reshape(-1, K)

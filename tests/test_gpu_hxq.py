@@ -328,3 +328,24 @@ def test_unaligned_contiguous_view(dev, dt, n):
     assert torch.equal(y, mod(x.clone()))
     ref = oracle.linear_f64(x.float().cpu().numpy(), _oracle_w(L))
     assert _maxrel(y.float().cpu().numpy(), ref) <= (TOL_F32 if dt == torch.float32 else TOL_BF16)
+
+
+@pytest.mark.parametrize("rows", [1, 16])
+def test_tensors_assigned_as_parameters(dev, rows):
+    """nn.Module moves a buffer's name to the parameters when a caller assigns one: the
+    kernels read it there."""
+    T = synth.to_torch(synth.make_layer_np(96, 256, seed=3))
+    m = HelixLinear(256, 96, T["codebook"], T["indices"], T["sidecar_positions"],
+                    T["sidecar_values"], bias=torch.linspace(-0.5, 0.5, 96),
+                    group_scale=T["group_scale"], group_offset=T["group_offset"],
+                    group_size=T["group_size"]).to(dev)
+    x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(rows)).to(dev)
+    print(f"parameters rows={rows}", flush=True)
+    with torch.no_grad():
+        y = m(x)
+        m.bias = torch.nn.Parameter(m.bias + 1, requires_grad=False)
+        m.codebook = torch.nn.Parameter(m.codebook.clone(), requires_grad=False)
+        assert "bias" not in m._buffers and "codebook" not in m._buffers
+        # one fp32 rounding of the sum with the bias on either side: 2 ulp of |y| + 2
+        bound = 2 * 2.0 ** -23 * (float(y.abs().max()) + 2)
+        assert float((m(x) - (y + 1)).abs().max()) <= bound
