@@ -80,7 +80,7 @@ Plan plan(int64_t m, int64_t out, int64_t in, bool f32, bool affine, int32_t gro
     p.mt = static_cast<int>((rows + kSub - 1) / kSub);
     double cost = 0;
     for (int ns : {1, 2, 3, 5}) {
-        if (ns > 3 && format == HXQ_FMT_SCALAR_U16) break;  // two index loads: registers
+        if (ns > kWideSubs && format == HXQ_FMT_SCALAR_U16) break;
         const int64_t blocks = (subs + ns - 1) / ns * by;
         const double c = static_cast<double>((blocks + cus - 1) / cus) * (ns * static_cast<double>(in) + 6000.0);
         if (ns == 1 || c < cost) {

@@ -554,6 +554,7 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
 }
 
 constexpr int kMaxRows = 64, kMaxRowsF32 = 32;
+constexpr int kWideSubs = 3;     // most subtiles per block with uint16 scalar indices (two index loads: registers)
 constexpr int kGroupedSubs = 5;  // subtiles per block of a grouped launch (16-row tiles)
 
 // Launches the kernel for XT with mt row tiles and ns subtiles per block.

@@ -10,20 +10,30 @@ namespace rw {
 
 template <int XT, int MT, int NS, int SP, int W>
 static int launch_fmt(const Call &c, int format, bool aff, const Plan &p, hipStream_t stream) {
-    const dim3 grid(p.bx, p.by), block(W * 64);
-#define HXQ_RW(AF_, F_) \
-    hipLaunchKernelGGL((rows_kernel<MT, NS, SP, XT, AF_, F_, W>), grid, block, 0, stream, c.idx, c.x, c.cb, \
-                       c.ga, c.M, c.OUT, c.K, c.ngroups, c.gmul, c.a, 0)
+    const dim3 grid(p.bx, p.by);
+#define HXQ_RW(AF_, F_, W_) \
+    hipLaunchKernelGGL((rows_kernel<MT, NS, SP, XT, AF_, F_, W_>), grid, dim3(W_ * 64), 0, stream, c.idx, c.x, \
+                       c.cb, c.ga, c.M, c.OUT, c.K, c.ngroups, c.gmul, c.a, 0)
     switch (format) {
         case HXQ_FMT_SCALAR:
-            if (aff) HXQ_RW(true, HXQ_FMT_SCALAR); else HXQ_RW(false, HXQ_FMT_SCALAR);
+            if (aff) HXQ_RW(true, HXQ_FMT_SCALAR, W); else HXQ_RW(false, HXQ_FMT_SCALAR, W);
             break;
         case HXQ_FMT_SCALAR_U16:
-            if (aff) HXQ_RW(true, HXQ_FMT_SCALAR_U16); else HXQ_RW(false, HXQ_FMT_SCALAR_U16);
+            if constexpr (NS <= kWideSubs) {
+                // two index loads and the affine: 16 waves leave 128 registers, which
+                // spill (36 and 44 bytes a lane at 1 x 1 x 4 and 2 x 3 x 1).  us with
+                // 16 / 8 waves: 16 x 18944 x 3584 40.7 / 35.0, 17 x 18944 x 3584
+                // 56.5 / 44.8, 16 x 3584 x 18944 48.3 / 40.2, 16 x 512 x 3584 10.0 /
+                // 10.3; two row tiles of one subtile fit 16: 17 x 3584 x 18944 41.3 / 43.3
+                constexpr int WA = MT == 2 && NS == 1 ? W : 8;
+                if (aff) HXQ_RW(true, HXQ_FMT_SCALAR_U16, WA); else HXQ_RW(false, HXQ_FMT_SCALAR_U16, W);
+            } else {
+                HXQ_REQUIRE(false, "no such few-row plan");
+            }
             break;
-        case HXQ_FMT_VQ2_U16: HXQ_RW(false, HXQ_FMT_VQ2_U16); break;
-        case HXQ_FMT_VQ2_P12: HXQ_RW(false, HXQ_FMT_VQ2_P12); break;
-        default: HXQ_RW(true, HXQ_FMT_AF6); break;
+        case HXQ_FMT_VQ2_U16: HXQ_RW(false, HXQ_FMT_VQ2_U16, W); break;
+        case HXQ_FMT_VQ2_P12: HXQ_RW(false, HXQ_FMT_VQ2_P12, W); break;
+        default: HXQ_RW(true, HXQ_FMT_AF6, W); break;
     }
 #undef HXQ_RW
     HXQ_LAUNCH_CHECK();
