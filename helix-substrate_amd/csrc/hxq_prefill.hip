@@ -944,6 +944,12 @@ Plan plan(int64_t m, int64_t out, int64_t in, int cus, int bm_max = 256) {
     return p;
 }
 
+// uint16 scalar indices with the affine need more registers than the 256-row
+// tile leaves; the fp32 A tile doubles the LDS: 128-row tiles.
+int max_bm(bool f32, int format, bool affine) {
+    return f32 || (format == HXQ_FMT_SCALAR_U16 && affine) ? 128 : 256;
+}
+
 bool grouped_ok(const hxq_expert_bank *b, int64_t out, int64_t in, int32_t group) {
     return b && b->indices && b->codebook && in % kBK == 0 && in < (int64_t{1} << 26) &&
            (!b->group_affine || (group >= kBK && group % kBK == 0 && in % group == 0)) &&
@@ -1095,14 +1101,26 @@ int grouped_gemm(const GroupedReq &r, hipStream_t stream) {
 
 using namespace hxq;
 
+extern "C" int64_t hxq_prefill_gemm_plan(int64_t m_rows, int64_t out_features, int64_t in_features,
+                                         int32_t x_dtype, int32_t format, int32_t group_size) {
+    if (m_rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % pg::kBK) return 0;
+    const int cus = device_cu_count();
+    const bool f32 = x_dtype == HXQ_F32;
+    if (rw::plan(m_rows, out_features, in_features, f32, group_size > 0, group_size, format, cus).mt > 0) return -1;
+    return pg::plan(m_rows, out_features, in_features, cus, pg::max_bm(f32, format, group_size > 0)).ws_bytes;
+}
+
 extern "C" int64_t hxq_prefill_gemm_workspace_bytes(int64_t m_rows, int64_t out_features,
                                                     int64_t in_features) {
-    if (m_rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % pg::kBK) return 0;
-    // the largest over the row-tile heights a format may use
-    if (m_rows <= rw::kMaxRows && in_features < 16384) return 0;  // the few-row kernel, every format and type
-    const int cus = device_cu_count();
-    return std::max(pg::plan(m_rows, out_features, in_features, cus).ws_bytes,
-                    pg::plan(m_rows, out_features, in_features, cus, 128).ws_bytes);
+    // the most that any type, format and group size takes: of these, the plans
+    // look at fp32 X, at uint16 indices with and without the affine, and at
+    // groups of 16384 columns and more that do not span K
+    int64_t most = 0;
+    for (int32_t x_dtype : {HXQ_BF16, HXQ_F32})
+        for (int32_t format : {HXQ_FMT_SCALAR, HXQ_FMT_SCALAR_U16})
+            for (int32_t group : {0, 16, 16384})
+                most = std::max(most, hxq_prefill_gemm_plan(m_rows, out_features, in_features, x_dtype, format, group));
+    return most;
 }
 
 extern "C" int hxq_prefill_gemm(const void *x, int32_t x_dtype, int32_t format,
@@ -1169,13 +1187,9 @@ extern "C" int hxq_prefill_gemm(const void *x, int32_t x_dtype, int32_t format,
         if (x_dtype == HXQ_F16) return rw::launch_rows<0>(r, format, aff, rp, stream);
         return rw::launch_rows<2>(r, format, aff, rp, stream);
     }
-    // uint16 scalar indices with the affine need more registers than the
-    // 256-row tile leaves: 128-row tiles
-    // fp32 activations: 128-row tiles (the fp32 A tile doubles the LDS)
-    const bool u16_aff = format == HXQ_FMT_SCALAR_U16 && group_affine != nullptr;
     const bool f32 = x_dtype == HXQ_F32;
     const pg::Plan p = pg::plan(m_rows, out_features, in_features, device_cu_count(),
-                                (u16_aff || f32) ? 128 : 256);
+                                pg::max_bm(f32, format, group_affine != nullptr));
     pg::Args a{};
     a.x = static_cast<const uint16_t *>(x);
     a.idx = indices;

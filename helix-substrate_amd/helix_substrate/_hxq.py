@@ -136,6 +136,7 @@ SIGNATURES_I64 = {
     "hxq_gemm_workspace_bytes": [I64, I64, I64],
     "hxq_gemm_noalloc_max_bytes": [],
     "hxq_prefill_gemm_workspace_bytes": [I64, I64, I64],
+    "hxq_prefill_gemm_plan": [I64, I64, I64, I32, I32, I32],
 }
 
 
@@ -493,9 +494,11 @@ def prefill_gemm(x, indices, codebook, group_affine, group_size, sc_grp_ptr, sc_
 
 def _prefill_call(L, x, m, out_f, in_f, fmt, indices, codebook, n_codes, group_affine, group_size,
                   sc_grp_ptr, sc_grp_key, sc_grp_val, bias, out):
-    nbytes = L.hxq_prefill_gemm_workspace_bytes(m, out_f, in_f)
+    xdt = dtype_code(x.dtype)
+    # -1: the few-row kernel, which takes no workspace
+    nbytes = L.hxq_prefill_gemm_plan(m, out_f, in_f, xdt, fmt, 0 if group_affine is None else int(group_size))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes > 0 else None
-    return L.hxq_prefill_gemm(_ptr(x), dtype_code(x.dtype), fmt, _ptr(indices), _ptr(codebook),
+    return L.hxq_prefill_gemm(_ptr(x), xdt, fmt, _ptr(indices), _ptr(codebook),
                               n_codes, _ptr(group_affine), int(group_size), _ptr(sc_grp_ptr),
                               _ptr(sc_grp_key), _ptr(sc_grp_val), _ptr(bias), _ptr(out),
                               dtype_code(out.dtype), m, out_f, in_f, _ptr(ws), nbytes, _stream(x))

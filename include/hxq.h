@@ -278,15 +278,21 @@ int hxq_gemm_ws(const void *x, int32_t x_dtype, const uint8_t *indices,
  * writes) for any group_size that is a positive multiple of 16; a caller
  * whose true K is not a multiple of 64 pads X and the index rows with zero
  * columns up to in_features and the affine with groups of (0, 0), so the
- * padded columns contribute nothing.  Shapes with few output tiles split K: a
- * workspace of hxq_prefill_gemm_workspace_bytes(...) bytes holds fp32
- * partials, reduced in order (deterministic).
+ * padded columns contribute nothing.  Two kernels: calls with few rows of X
+ * run one that needs no workspace; of the others, shapes with few output
+ * tiles split K, and a workspace holds fp32 partials, reduced in order (both
+ * deterministic).  hxq_prefill_gemm_plan says which: -1 is the few-row
+ * kernel, else the bytes of workspace of that call (group_size 0: no affine).
+ * hxq_prefill_gemm_workspace_bytes is the most that any activation type,
+ * format and group size needs at these sizes.
  * Replaces: fused_vq_matmul's N > 1 path (triton_vq_matmul.py:249-334,
  * 634-661, 693-698, 724-725) and HelixLinear._forward_buffered
  * (helix_linear.py:556-634).
  */
 int64_t hxq_prefill_gemm_workspace_bytes(int64_t m_rows, int64_t out_features,
                                          int64_t in_features);
+int64_t hxq_prefill_gemm_plan(int64_t m_rows, int64_t out_features, int64_t in_features,
+                              int32_t x_dtype, int32_t format, int32_t group_size);
 int hxq_prefill_gemm(const void *x, int32_t x_dtype, int32_t format, const uint8_t *indices,
                      const float *codebook, int32_t n_codes, const float *group_affine,
                      int32_t group_size,

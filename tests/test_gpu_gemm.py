@@ -138,7 +138,7 @@ def test_prefill_sidecar_dense_block_and_repeats(dev):
     """A 64 x 64 block fully in the sidecar (4096 entries in one row group and
     K step: the per-step list overflows its 64-entry load), positions repeated
     with new values (the last copy wins), under a K split."""
-    out_f, in_f, m = 256, 512, 96
+    out_f, in_f, m = 1000, 512, 1001   # the tiled kernel
     L = synth.make_layer_np(out_f, in_f, seed=21, sidecar=False)
     rs = np.random.RandomState(3)
     blk = (np.arange(64, 128)[:, None] * in_f + np.arange(128, 192)[None, :]).ravel()
@@ -152,7 +152,7 @@ def test_prefill_sidecar_dense_block_and_repeats(dev):
     W = _oracle_w(L)
     assert np.array_equal(W.exact.ravel()[rep], val[-50:])   # the last copy is the oracle's value
     x = torch.randn(m, in_f, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16)
-    assert _hxq.lib().hxq_prefill_gemm_workspace_bytes(m, out_f, in_f) > 0   # K is split
+    assert _hxq.lib().hxq_prefill_gemm_plan(m, out_f, in_f, 1, _hxq.FMT_SCALAR, 128) > 0   # K is split
     _check(_gemm32(mod, x.to(dev)), x, W)
     y = mod(x.to(dev))
     assert mod._last_dispatch_path == "hip_gemm"

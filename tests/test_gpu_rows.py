@@ -117,3 +117,19 @@ def test_rows_grouped(dev, counts, out, inp, xdt):
         W16 = torch.from_numpy(W).to(xdt).float().numpy()
         ref = oracle.linear_np(x[rows[lo:hi].long()].float().numpy(), W16)
         assert _maxrel(y[lo:hi], ref) <= 2e-5, e   # operands equal: order of fp32 sums
+
+
+def test_rows_allocate_nothing(dev):
+    """A few-row call into a given output allocates no workspace, whatever K is."""
+    m, out, inp = 16, 512, 18944
+    idx = torch.randint(0, 256, (out, inp), dtype=torch.uint8, device=dev)
+    cb = torch.randn(256, device=dev)
+    x = torch.randn(m, inp, device=dev).to(torch.bfloat16)
+    y = torch.empty(m, out, dtype=torch.bfloat16, device=dev)
+    args = (x, idx, cb, None, 128, None, None, None)
+    _hxq.prefill_gemm(*args, out=y)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    _hxq.prefill_gemm(*args, out=y)
+    assert torch.cuda.max_memory_allocated() == before

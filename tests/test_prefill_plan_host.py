@@ -1,0 +1,41 @@
+"""Which kernel a prefill GEMM call runs and what workspace it takes (hxq_prefill_gemm_plan), and
+the bound over all types and formats.  No GPU: the plans count on 256 compute units then."""
+import pytest
+
+from helix_substrate import _hxq
+from helix_substrate._hxq import FMT_SCALAR, FMT_SCALAR_U16, FMT_VQ2_P12
+
+BF16, F32 = 1, 0
+
+
+def plan(m, out, k, dt=BF16, fmt=FMT_SCALAR, group=128):
+    return _hxq.lib().hxq_prefill_gemm_plan(m, out, k, dt, fmt, group)
+
+
+def test_dtype_codes():
+    import torch
+    assert (_hxq.dtype_code(torch.float32), _hxq.dtype_code(torch.bfloat16)) == (F32, BF16)
+
+
+@pytest.mark.parametrize("m,out,k", [(16, 3584, 18944), (64, 3584, 18944), (80, 8512, 2048),
+                                     (512, 512, 3584), (5, 256, 256)])
+def test_few_row_calls_take_no_workspace(m, out, k):
+    assert plan(m, out, k) == -1
+    if m <= 64:
+        assert plan(m, out, k, F32) == -1
+
+
+@pytest.mark.parametrize("m,out,k", [(m, out, k) for m in (1, 16, 64, 65, 128, 129, 300, 1001, 8192)
+                                     for out in (16, 512, 1000, 3584, 18944)
+                                     for k in (64, 512, 2048, 18944, 32768)])
+def test_bound_covers_every_type_and_format(m, out, k):
+    most = _hxq.lib().hxq_prefill_gemm_workspace_bytes(m, out, k)
+    plans = [plan(m, out, k, dt, fmt, g) for dt in (BF16, 2, F32)
+             for fmt in (FMT_SCALAR, FMT_SCALAR_U16, FMT_VQ2_P12) for g in (0, 16, 128, 16384)
+             if not (fmt == FMT_VQ2_P12 and g)]
+    assert most == max(0, max(plans))
+
+
+def test_tiled_plan_splits_k():
+    assert plan(1001, 1000, 512) > 0        # 32 tiles of 128 x 256, K in two ranges
+    assert plan(8192, 8192, 3584) == 0      # 1024 tiles of 256 x 256: whole rounds, no split
