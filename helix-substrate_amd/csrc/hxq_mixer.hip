@@ -48,21 +48,23 @@ __device__ __forceinline__ void st16or32(void *p, int64_t i, int dt, float v) {
     else static_cast<uint16_t *>(p)[i] = f32_to_f16(v);
 }
 
-// v / (1 + exp(-v)) to within an ulp or two in 14 instructions (the library
-// exponential and an IEEE division take 30, and bounded the convolution and
-// the gated norm: 110 us for 71M values): exp2 of -v log2(e) in two parts, the
-// hardware reciprocal with one Newton step.  -v is held to where the
-// exponential is finite; below -86 (sums over 2e37, whose reciprocal is
-// denormal) the plain reciprocal gives the limit -0.
+// v / (1 + exp(-v)), the same bits as that expression gives for every fp32 v.
+// In the middle range the IEEE division is the hardware reciprocal with one
+// Newton step and the quotient's residual (6 instructions against 10); outside
+// it, where quotient or reciprocal come near the ends of the exponent range,
+// v is 0, infinite or NaN, the division itself.  Both forms compared over all
+// 2^32 patterns of v: no bit differs.  Convolution of 8 x 2048 tokens, 4352
+// channels: 107.8 us, 128.8 with the division.
 __device__ __forceinline__ float silu(float v) {
-    const float w = -fminf(fmaxf(v, -88.7f), 100.f);
-    const float p = w * 1.44269502f;
-    const float lo = fmaf(w, 1.92596299e-8f, fmaf(w, 1.44269502f, -p));
-    float e = __builtin_amdgcn_exp2f(p);
-    e = fmaf(e, lo * 0.693147182f, e);
-    const float d = 1.f + e;
-    const float r = __builtin_amdgcn_rcpf(d);
-    return v * (d < 2e37f ? fmaf(fmaf(-d, r, 1.f), r, r) : r);
+    const float d = 1.f + expf(-v);
+    const float a = fabsf(v);
+    if (a > 0x1p-60f && a < 60.f) {
+        float r = __builtin_amdgcn_rcpf(d);
+        r = fmaf(fmaf(-d, r, 1.f), r, r);
+        const float q = v * r;
+        return fmaf(fmaf(-d, q, v), r, q);
+    }
+    return v / d;
 }
 
 // Two fp32 values rounded to nearest even in one conversion.
@@ -160,8 +162,8 @@ __global__ __launch_bounds__(256) void conv_split_kernel(const ConvArgs a) {
 // 16-byte store; the W-1 previous inputs of its channels stay in registers
 // (W <= 4).  The grid's last column of blocks does the dt channels.  Bound by
 // memory latency and the SiLU's arithmetic: 8 x 2048 tokens of 4352 channels
-// 152 to 97 us with the short silu() above, the taps by way of LDS, the next
-// round's rows requested ahead and the dt channels in the same launch.
+// 152 to 108 us with the silu() above, the taps by way of LDS, the next round's
+// rows requested ahead and the dt channels in the same launch.
 template <int W, bool BF16>
 __global__ __launch_bounds__(256) void conv_split_vec_kernel(const ConvArgs a) {
     const int conv_dim = a.d_inner + 2 * a.gn;

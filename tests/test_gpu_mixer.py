@@ -66,6 +66,35 @@ def test_conv_step_matches_prefill(dev):
         assert torch.allclose(dts, dt[:, t], rtol=1e-6, atol=1e-6)
 
 
+def test_silu_over_its_whole_range(dev):
+    """The SiLU of the convolution, value by value, from where the exponential overflows to where
+    it vanishes.  Bound: 1 ulp for the exponential, half an ulp each for the sum and the
+    quotient, 2^-23 relative an ulp."""
+    n = 1 << 16
+    v = np.concatenate([np.linspace(-88.7, -87.0, 4096), np.linspace(-88.7, 100.0, n - 4096 - 256),
+                        np.geomspace(1e-37, 1.0, 128), -np.geomspace(1e-37, 1.0, 128)])
+    v = v.astype(np.float32)
+    proj = torch.from_numpy(v).reshape(n // 64, 1, 64)
+    w = torch.tensor([[0.0, 0.0, 0.0, 1.0]]).expand(64, 4).contiguous()
+    # 64 channels: 32 of x, 16 each of B and C; the dt of 1 head is column 0 again
+    args = (None, None, 0.0, float("inf"), 0, 32, 1, 16, 1)
+    padded = torch.cat([torch.zeros(n // 64, 1, 32), proj, torch.zeros(n // 64, 1, 1)], dim=2)
+    out = _hxq.mamba2_conv_split(padded.to(dev), w.to(dev), *args, out_dtype=torch.float32)
+    got = torch.cat([t.reshape(n // 64, -1) for t in out[:3]], dim=1).cpu().numpy().ravel()
+    d = v.astype(np.float64)
+    ref = d / (1.0 + np.exp(-d))
+    assert np.abs(got / ref - 1.0).max() <= 2.0 ** -22
+    lim = torch.tensor([-float("inf"), float("inf"), float("nan"), -1e4]).repeat(16).reshape(1, 1, 64)
+    cs = torch.zeros(1, 64, 4, device=dev)
+    padded = torch.cat([torch.zeros(1, 1, 32), lim, torch.zeros(1, 1, 1)], dim=2)[:, 0].contiguous()
+    one = torch.ones(64, 1, device=dev)   # one tap: no 0 * inf
+    out = _hxq.mamba2_conv_step(padded.to(dev), cs[:, :, :1].contiguous(), one, *args,
+                                out_dtype=torch.float32)
+    got = torch.cat([t.reshape(-1) for t in out[:3]]).cpu().reshape(16, 4)
+    assert torch.isnan(got[:, 0]).all() and torch.isnan(got[:, 2]).all()   # -inf / inf
+    assert torch.isposinf(got[:, 1]).all() and (got[:, 3] == 0).all()
+
+
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 def test_gated_rmsnorm_matches_oracle(dev, gdt):
     rows, width, stride = 33, 1000, 1300
