@@ -55,15 +55,24 @@ namespace rw {
 
 // The few-row plan of a call (mt 0: the tiled kernel runs).
 //
-// Where the line lies: up to 128 rows (two blocks of 64 per run of W) always,
-// above that while the 16-row subtiles of W times the 64-row blocks of X stay
-// within three per CU, two where K is above 8192 (X is read again by every
-// block).  Measured, us, tiled against few-row: 16 x 18944 x 3584 (M, OUT, K)
-// 60.1 / 24.2, 16 x 3584 x 18944 70.0 / 29.6, 64 x 18944 x 3584 61.5 / 33.8,
-// 64 x 3584 x 18944 71.1 / 50.5, 128 x 8512 x 2048 40.2 / 23.0, 512 x 512 x
-// 3584 23.1 / 14.4, 192 x 3584 x 3584 28.0 / 24.4; past the line 256 x 3584 x
-// 3584 28.9 / 32.4, 512 x 2048 x 4096 32.3 / 35.2.  fp32 X (32-row blocks):
-// 16 x 18944 x 3584 174 / 38.6, 64 x 3584 x 3584 69.5 / 26.7.
+// Where the line lies.  Up to 64 rows of X (fp32: 32) one block per run of W:
+// always.  Above that W is dequantised and X read once more for every block of
+// rows, and the work is the 16-row subtiles of W times the row blocks, counted
+// per CU.  Measured, us, tiled / few-row:
+//   one row block: 16 x 18944 x 3584 (M, OUT, K) 60.1 / 24.2, 64 x 18944 x 3584
+//   61.5 / 33.8, 64 x 3584 x 18944 71.1 / 50.5, fp32 16 x 18944 x 3584 177 / 40;
+//   two: up to 6 per CU, 65 rows of 11008 x 2048 33.7 / 28.5, 10240 x 8192
+//   70.4 / 64.7, 6144 x 16384 89.0 / 80.8, 3584 x 18944 72.5 / 63.5; past it
+//   14336 x 4096 55.4 / 65.0, 18944 x 18944 255.9 / 280.9 (96 rows), 18944 x
+//   3584 no difference (63.0 / 62.1; 128 rows 64.5 / 65.1); 12-bit pairs alike.
+//   uint16 indices, at most three subtiles a block and so more rounds: 4.5 per
+//   CU, 9216 x 3584 54.1 / 44.6, 8512 x 2048 32.4 / 30.0, past it 10240 x 2048
+//   27.1 / 30.9, 18944 x 3584 59.7 / 89.3; 2 with K above 8192, 3584 x 18944
+//   90.6 / 75.1, past it 6144 x 16384 76.4 / 87.3.  fp32 X: no end to it, 33 x
+//   18944 x 3584 173 / 106, 33 x 3584 x 18944 320 / 111;
+//   more: 3 per CU, 2 with K above 8192: 512 x 512 x 3584 23.1 / 14.4, 192 x 3584
+//   x 3584 30.9 / 27.3, fp32 128 x 3072 x 3584 76.2 / 40.7, past it 256 x 3584 x
+//   3584 28.9 / 32.4, 512 x 2048 x 4096 32.3 / 35.2.
 //
 // Subtiles per block: one block runs per CU, so a block count is rounds of the
 // chip, and each round costs a fixed part (table, first loads, final sum: the
@@ -74,13 +83,19 @@ Plan plan(int64_t m, int64_t out, int64_t in, bool f32, bool affine, int32_t gro
     const int64_t most = f32 ? kMaxRowsF32 : kMaxRows;
     const int64_t by = (m + most - 1) / most;
     const int64_t subs = (out + kSub - 1) / kSub;
-    if (by > 2 && subs * by > (in > 8192 ? 2 : 3) * cus) return p;
+    const bool u16 = format == HXQ_FMT_SCALAR_U16;
+    const int64_t halves = by <= 1 || (by == 2 && f32) ? 0              // of a CU's subtiles; 0: any number
+                           : by == 2 && !u16           ? 12
+                           : in > 8192                 ? 4
+                           : by == 2                   ? 9
+                                                       : 6;
+    if (halves && 2 * subs * by > halves * cus) return p;
     const int64_t rows = (m + by - 1) / by;
     p.by = static_cast<int>(by);
     p.mt = static_cast<int>((rows + kSub - 1) / kSub);
     double cost = 0;
     for (int ns : {1, 2, 3, 5}) {
-        if (ns > kWideSubs && format == HXQ_FMT_SCALAR_U16) break;
+        if (ns > kWideSubs && u16) break;
         const int64_t blocks = (subs + ns - 1) / ns * by;
         const double c = static_cast<double>((blocks + cus - 1) / cus) * (ns * static_cast<double>(in) + 6000.0);
         if (ns == 1 || c < cost) {

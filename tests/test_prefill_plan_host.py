@@ -39,3 +39,21 @@ def test_bound_covers_every_type_and_format(m, out, k):
 def test_tiled_plan_splits_k():
     assert plan(1001, 1000, 512) > 0        # 32 tiles of 128 x 256, K in two ranges
     assert plan(8192, 8192, 3584) == 0      # 1024 tiles of 256 x 256: whole rounds, no split
+
+
+@pytest.mark.parametrize("fmt,dt,few,tiled", [
+    # two row blocks of X: W's subtiles times the row blocks, per CU, decide
+    (FMT_SCALAR, BF16, [(65, 11008, 2048), (128, 10240, 8192), (128, 6144, 16384), (65, 3584, 18944)],
+     [(65, 14336, 4096), (128, 14336, 4096), (96, 18944, 18944)]),
+    (FMT_VQ2_P12, 2, [(65, 11008, 2048), (128, 6144, 16384)], [(65, 14336, 4096)]),
+    (FMT_SCALAR_U16, BF16, [(65, 9216, 3584), (128, 8512, 2048), (65, 3584, 18944)],
+     [(65, 10240, 2048), (65, 10240, 8192), (128, 18944, 3584), (65, 6144, 16384)]),
+    (FMT_SCALAR_U16, F32, [(33, 18944, 3584), (64, 6144, 16384)], []),
+    (FMT_SCALAR, F32, [(33, 18944, 3584), (64, 3584, 18944)], []),
+])
+def test_line_between_the_kernels(fmt, dt, few, tiled):
+    group = 0 if fmt == FMT_VQ2_P12 else 128
+    for s in few:
+        assert plan(*s, dt, fmt, group) == -1, s
+    for s in tiled:
+        assert plan(*s, dt, fmt, group) >= 0, s
