@@ -973,9 +973,38 @@ bool grouped_ok(const hxq_expert_bank *b, int64_t out, int64_t in, int32_t group
            (!b->group_affine || (in / group) * out * 8 < (int64_t{1} << 31));
 }
 
-#ifndef GRP_BM64_MAX
-#define GRP_BM64_MAX 96
-#endif
+// Height of a grouped launch's row tiles: 16 is the few-row kernel, else the
+// tiled one with 256-row tiles when the experts average more than 192 rows, 128
+// above 96, else 64 (fp32 activations: 128 always, the fp32 A tile doubles the
+// LDS).
+//
+// Where the few-row line lies: an expert with more than 16 rows has W dequantised
+// once per 16 of them, which a tile of 64 does once, and the routing that decides
+// it is on the device.  So the line holds for uneven routing too: at most 12
+// rows per expert on average, and 48 / sqrt(n_exp), since with more experts the
+// 64-row tiles fill the chip by themselves and gain less is to be had.  Whole FFN,
+// us, 64-row tiles / few-row, with routing that is even / favours top_k experts /
+// favours a quarter of the experts / takes top_k experts only:
+//   64 experts, top 8, 2048 -> 1024: 4 tokens 97 / 76, 96 / 59, -, 92 / 47; 16
+//   143 / 129, 131 / 92, -, 93 / 47; 48 151 / 147, 144 / 146, 137 / 139, 93 / 74;
+//   past the line 56 147 / 145, 142 / 159, 137 / 141, 91 / 86; 80 151 / 146,
+//   149 / 175, -, 97 / 99;
+//   64, top 8, 4096 -> 1536: 48 tokens 414 / 366, 380 / 361, 358 / 331, 146 / 136;
+//   past it 64 408 / 348, 386 / 400, 367 / 357, 147 / 165;
+//   128, top 8, 2048 -> 768: 64 tokens 218 / 208, 200 / 203, 120 / 107, 86 / 75;
+//   past it 80 230 / 214, 204 / 217, 122 / 139, 87 / 86;
+//   32, top 4, 2048 -> 1024: 64 tokens 98 / 87, 96 / 90, 95 / 89, 90 / 56; past
+//   it 80 97 / 87, 96 / 102, 94 / 100, 89 / 69;
+//   16, top 2, 2048 -> 4096: 96 tokens 194 / 150, 189 / 174, 187 / 178, 154 / 102;
+//   8, top 2, 4096 -> 14336: 48 tokens 628 / 404, 627 / 537, 627 / 529, 608 / 288.
+int grouped_bm(int64_t n_assign, int64_t n_exp, int x_dtype, int64_t out, int32_t group) {
+    if (x_dtype == HXQ_F32) return 128;
+    if (n_assign <= 12 * n_exp && n_assign * n_assign <= 48 * 48 * n_exp && out % 4 == 0 && group < 16384)
+        return rw::kSub;
+    const int64_t mean_rows = n_assign / n_exp;
+    return mean_rows > 192 ? 256 : mean_rows > 96 ? 128 : 64;
+}
+
 int grouped_gemm(const GroupedReq &r, hipStream_t stream) {
     HXQ_REQUIRE(r.x && r.seg && r.bank0 && r.y, "x, expert_offsets, bank and y are required");
     HXQ_REQUIRE(r.x_dtype == HXQ_BF16 || r.x_dtype == HXQ_F16 || r.x_dtype == HXQ_F32,
@@ -996,14 +1025,9 @@ int grouped_gemm(const GroupedReq &r, hipStream_t stream) {
                     (reinterpret_cast<uintptr_t>(r.bank0->indices) & 15u) == 0 &&
                     (!r.bank1 || (reinterpret_cast<uintptr_t>(r.bank1->indices) & 15u) == 0),
                 "x and indices must be 16-byte aligned");
-    // Experts that average at most 12 rows run the few-row kernel in 16-row
-    // tiles.  Whole FFN of 64 experts (top 8, 2048 -> 1024), us, 64-row tiles
-    // against few-row: 1 token 87.5 / 43.4, 4 96.4 / 76.4, 16 140.9 / 125.9,
-    // 64 147.9 / 143.8; 100 tokens on 32 experts, top 4 (12 rows) 98.1 / 91.5;
-    // past the line (128 tokens, 16 rows: two tiles for many) 153.3 / 185.5.
+    const int bm = grouped_bm(r.n_assign, r.n_exp, r.x_dtype, r.out0, r.bank0->group_affine ? r.group : 0);
     const bool aff_bank = r.bank0->group_affine != nullptr;
-    if (r.x_dtype != HXQ_F32 && r.n_assign <= 12 * static_cast<int64_t>(r.n_exp) && r.out0 % 4 == 0 &&
-        (!aff_bank || r.group < 16384) && (reinterpret_cast<uintptr_t>(r.y) & 15u) == 0) {
+    if (bm == rw::kSub && (reinterpret_cast<uintptr_t>(r.y) & 15u) == 0) {
         rw::Grouped q{};
         auto fill = [&](const hxq_expert_bank *b, rw::Bank &o) {
             o.idx = b->indices;
@@ -1081,13 +1105,11 @@ int grouped_gemm(const GroupedReq &r, hipStream_t stream) {
     a.cb_es = 256;
     a.ga_es = aff ? (r.in / a.group) * wo : 0;
     a.scp_es = (wo + 63) / 64 * (r.in / kBK) + 1;
-    // 256-row tiles when the experts average more than 192 rows, 128 above 96, else 64
-    // (fp32 activations: 128-row tiles always, the fp32 A tile doubles the LDS)
-    const int64_t mean_rows = r.n_assign / r.n_exp;
     const bool f32 = r.x_dtype == HXQ_F32;
-    const int bm = f32 ? 128 : mean_rows > 192 ? 256 : mean_rows > GRP_BM64_MAX ? 128 : 64;
     a.grp_tiles_x = static_cast<int32_t>((out + kBN - 1) / kBN);
-    const int64_t row_tiles = (r.n_assign + bm - 1) / bm + r.n_exp;  // upper bound over any routing
+    // (16-row tiles that y's alignment rules out run as 64)
+    const int bt = std::max(bm, 64);
+    const int64_t row_tiles = (r.n_assign + bt - 1) / bt + r.n_exp;  // upper bound over any routing
     a.grp_per_xcd = static_cast<int32_t>((row_tiles + kXcds - 1) / kXcds * a.grp_tiles_x);
     const dim3 grid(static_cast<uint32_t>(a.grp_per_xcd) * kXcds);
     const bool bf16 = r.x_dtype == HXQ_BF16;
@@ -1096,10 +1118,10 @@ int grouped_gemm(const GroupedReq &r, hipStream_t stream) {
                        dim3(kBN / (32 * kNJ) * 64), 0, stream, a)
     if (f32) {
         if (aff) HXQ_PG_GRP(128, 2, true); else HXQ_PG_GRP(128, 2, false);
-    } else if (bm == 256) {
+    } else if (bt == 256) {
         if (bf16) { if (aff) HXQ_PG_GRP(256, 1, true); else HXQ_PG_GRP(256, 1, false); }
         else { if (aff) HXQ_PG_GRP(256, 0, true); else HXQ_PG_GRP(256, 0, false); }
-    } else if (bm == 64) {
+    } else if (bt == 64) {
         if (bf16) { if (aff) HXQ_PG_GRP(64, 1, true); else HXQ_PG_GRP(64, 1, false); }
         else { if (aff) HXQ_PG_GRP(64, 0, true); else HXQ_PG_GRP(64, 0, false); }
     } else {
@@ -1115,6 +1137,12 @@ int grouped_gemm(const GroupedReq &r, hipStream_t stream) {
 }  // namespace hxq
 
 using namespace hxq;
+
+extern "C" int hxq_moe_grouped_tile(int64_t n_assign, int32_t n_experts, int32_t x_dtype, int64_t out_features,
+                                    int32_t group_size) {
+    if (n_assign <= 0 || n_experts <= 0 || out_features <= 0) return 0;
+    return pg::grouped_bm(n_assign, n_experts, x_dtype, out_features, group_size);
+}
 
 extern "C" int64_t hxq_prefill_gemm_plan(int64_t m_rows, int64_t out_features, int64_t in_features,
                                          int32_t x_dtype, int32_t format, int32_t group_size) {

@@ -102,6 +102,7 @@ SIGNATURES = {
     "hxq_attn_rope_decode": [P, P, I32, I32, I32, F32, P, P, I32, I32, P, I32, P],
     "hxq_dense_gemv_bf16": [P, P, I32, I64, I64, P, P],
     "hxq_argmax": [P, I64, P, P, P, P],
+    "hxq_moe_grouped_tile": [I64, I32, I32, I64, I32],
     "hxq_moe_grouped_gemm": [P, I32, I64, P, P, I64, I32, P, I32, P, I32, I64, I64, P],
     "hxq_moe_ffn": [P, I32, I64, I64, I64, I32, I32, P, P, P, P, P, P, P, I32, P, I64, P, I32, P],
     "hxq_assign_nearest": [P, I64, P, I32, P, P],

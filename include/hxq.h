@@ -388,7 +388,12 @@ int hxq_moe_route(const float *logits, int64_t n_tokens, int32_t n_experts, int3
  * indices; banks with sc_grp_*) or into LDS as in hxq_gemm (otherwise).
  * Replaces: HelixLinear.forward per expert (helix_linear.py:318-361) on that
  * expert's token rows.
+ * hxq_moe_grouped_tile: the height of the row tiles (rows of one expert that
+ * share a dequantised W) that such a call runs with: 16 (the few-row kernel; y
+ * 16-byte aligned), 64, 128 or 256.  group_size 0: no affine.
  */
+int hxq_moe_grouped_tile(int64_t n_assign, int32_t n_experts, int32_t x_dtype,
+                         int64_t out_features, int32_t group_size);
 int hxq_moe_grouped_gemm(const void *x, int32_t x_dtype, int64_t x_rows,
                          const int32_t *sorted_rows, const int32_t *expert_offsets,
                          int64_t n_assign, int32_t n_experts, const hxq_expert_bank *bank,

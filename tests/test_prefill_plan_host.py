@@ -57,3 +57,21 @@ def test_line_between_the_kernels(fmt, dt, few, tiled):
         assert plan(*s, dt, fmt, group) == -1, s
     for s in tiled:
         assert plan(*s, dt, fmt, group) >= 0, s
+
+
+@pytest.mark.parametrize("experts,top_k,few,tiled", [
+    (8, 2, (1, 16, 48), (49,)), (16, 2, (4, 96), (97, 112)), (32, 4, (8, 64), (80, 96)),
+    (64, 8, (1, 4, 16, 48), (56, 64, 96)), (128, 8, (4, 64), (80,)), (256, 8, (8, 64), (97,)),
+])
+def test_grouped_line_holds_for_uneven_routing(experts, top_k, few, tiled):
+    """Tokens up to which 16-row tiles are no slower than 64-row ones, however few experts they go to."""
+    tile = _hxq.lib().hxq_moe_grouped_tile
+    for t in few:
+        assert tile(t * top_k, experts, BF16, 2048, 128) == 16, t
+        assert tile(t * top_k, experts, F32, 2048, 128) == 128
+        assert tile(t * top_k, experts, BF16, 2046, 128) == 64   # no whole 16-byte rows of Y
+        assert tile(t * top_k, experts, BF16, 2048, 16384) == 64
+    for t in tiled:
+        assert tile(t * top_k, experts, BF16, 2048, 128) == 64, t
+    assert tile(97 * experts, experts, BF16, 2048, 128) == 128
+    assert tile(193 * experts, experts, BF16, 2048, 128) == 256
