@@ -52,6 +52,22 @@ _CPU_TILE_ROWS = 256
 _GEMV_MAX_ROWS = 4
 _GEMV_MULTI_ROW_MAX_K = 8192  # 2-4 row GEMV launches hold 8 K-chunks of 1024 per wave
 
+# the tensors that the GPU forward reads
+_FORWARD_TENSORS = frozenset((
+    "indices", "_kidx", "codebook", "group_scale", "group_offset", "_affine_t", "bias",
+    "channel_scales", "_sc_row_ptr", "_sc_col", "_sc_delta", "_sc_grp_ptr", "_sc_grp_key",
+    "_sc_grp_val", "svd_U", "svd_s", "svd_Vt"))
+
+
+class _ByAttribute:
+    """A module's tensors by name, each looked up as an attribute when it is asked for."""
+
+    def __init__(self, module: nn.Module):
+        self._module = module
+
+    def __getitem__(self, name: str):
+        return getattr(self._module, name)
+
 
 class HelixLinear(nn.Module):
     """``y = x @ W^T + bias`` with W stored as codebook + uint8 indices (+ affine, sidecar).
@@ -319,13 +335,14 @@ class HelixLinear(nn.Module):
             padded = pad_columns(self.indices, self._kin // 2)
         self.register_buffer("_kidx", padded.contiguous(), persistent=False)
 
-    def _kernel_rows(self, x2: torch.Tensor, need: int):
+    def _kernel_rows(self, x2: torch.Tensor, need: int, tensors=None):
         """(activations, index rows) for a kernel whose K must be a multiple of
         `need` (16: GEMV, 64: GEMM): the stored layout when in_features is one,
         else the padded copy and x padded with zero columns."""
+        b = self._tensors() if tensors is None else tensors
         if self.in_features % need == 0:
-            return x2, self._tensors()["indices"]
-        return pad_columns(x2, self._kin), self._tensors()["_kidx"]
+            return x2, b["indices"]
+        return pad_columns(x2, self._kin), b["_kidx"]
 
     def _pair_index_at(self, rows: torch.Tensor, pairs: torch.Tensor) -> torch.Tensor:
         """Pair index at (row, pair column), from int16 or 12-bit packed storage."""
@@ -350,12 +367,14 @@ class HelixLinear(nn.Module):
 
     @property
     def _kcb(self) -> torch.Tensor:
+        return self._kernel_codebook(self.codebook)
+
+    def _kernel_codebook(self, cb: torch.Tensor) -> torch.Tensor:
         """The codebook as the scalar kernels read it: fp32 [256] (uint8 indices reach every
         entry).  A 256-entry fp32 codebook is used as is; a shorter one gets a zero-padded
         copy, rebuilt whenever the codebook tensor, its contents version or its device
         changes (e.g. after load_state_dict or .to()).  Codebooks above 256 entries
         (int16 indices) are read as they are: those kernels take the entry count."""
-        cb = self._tensors()["codebook"]
         if cb.dtype == torch.float32 and cb.numel() == 256 and cb.is_contiguous():
             return cb
         if cb.numel() > 256:
@@ -418,8 +437,6 @@ class HelixLinear(nn.Module):
         """Return ``x @ W^T + bias`` in x's dtype (reference helix_linear.py:318-361)."""
         input_dtype = x.dtype
         if x.is_cuda:
-            if not self._tensors()["codebook"].is_cuda:
-                raise RuntimeError("HelixLinear buffers are on the CPU but the input is on the GPU")
             out = self._forward_hip(x)
         elif getattr(self, "_wave_enabled", False):
             self._last_dispatch_path = "wave"
@@ -431,16 +448,20 @@ class HelixLinear(nn.Module):
             out = out.to(input_dtype)
         return out
 
-    def _tensors(self) -> dict:
-        """The tensors by name: the buffers' dict, with whatever a caller has assigned as a
-        Parameter (nn.Module moves that name out of the buffers; `weight` is one always)."""
-        p = self._parameters
-        return self._buffers if len(p) <= 1 else {**self._buffers, **p}
+    def _tensors(self):
+        """The forward's tensors by name: the buffers' dict while it holds them all (0.3 us to
+        see, what one attribute lookup of nn.Module takes), else by attribute lookup: a caller
+        may have assigned a Parameter or a plain attribute to a name, or parametrized it, and
+        nn.Module then keeps it elsewhere."""
+        b = self._buffers
+        return b if b.keys() >= _FORWARD_TENSORS else _ByAttribute(self)
 
     def _forward_hip(self, x: torch.Tensor) -> torch.Tensor:
-        # the buffers by their dict: nn.Module's attribute lookup is 0.3 us each,
-        # a third of a call whose kernel takes 5 us
+        # nn.Module's attribute lookups are a third of a call whose kernel takes 5 us
         b = self._tensors()
+        codebook = b["codebook"]
+        if not codebook.is_cuda:
+            raise RuntimeError("HelixLinear buffers are on the CPU but the input is on the GPU")
         orig_shape = x.shape
         K = self.in_features
         x2 = x if x.dim() == 2 and orig_shape[1] == K else x.reshape(-1, K)
@@ -466,15 +487,15 @@ class HelixLinear(nn.Module):
             # registers (bf16/fp16 MFMA for 16-bit activations, fp32 MFMA for
             # fp32 ones)
             self._last_dispatch_path = "hip_gemm"
-            xk, idx = self._kernel_rows(x2, 64)
-            _hxq.prefill_gemm(xk, idx, self._kcb if fmt == _hxq.FMT_SCALAR else b["codebook"],
-                              b["_affine_t"], self.group_size,
+            xk, idx = self._kernel_rows(x2, 64, b)
+            cb = self._kernel_codebook(codebook) if fmt == _hxq.FMT_SCALAR else codebook
+            _hxq.prefill_gemm(xk, idx, cb, b["_affine_t"], self.group_size,
                               b["_sc_grp_ptr"] if sidecar else None,
                               b["_sc_grp_key"] if sidecar else None,
                               b["_sc_grp_val"] if sidecar else None, b["bias"], out=out,
                               fmt=fmt, out_features=self.out_features)
         else:
-            xk, idx = self._kernel_rows(x2, 16)
+            xk, idx = self._kernel_rows(x2, 16, b)
             rp, col, delta = ((b["_sc_row_ptr"], b["_sc_col"], b["_sc_delta"]) if sidecar
                               else (None, None, None))
             self._last_dispatch_path = "hip_gemv" if fmt == _hxq.FMT_SCALAR else "hip_gemv_fmt"
@@ -482,13 +503,13 @@ class HelixLinear(nn.Module):
             for r0, r1 in groups:
                 xs, ys = (xk, out) if len(groups) == 1 else (xk[r0:r1], out[r0:r1])
                 if fmt != _hxq.FMT_SCALAR:
-                    _hxq.gemv_fmt(xs, fmt, idx, self.out_features, codebook=b["codebook"],
+                    _hxq.gemv_fmt(xs, fmt, idx, self.out_features, codebook=codebook,
                                   group_scale=b["group_scale"], group_offset=b["group_offset"],
                                   group_size=self.group_size, sc_row_ptr=rp, sc_col=col,
                                   sc_delta=delta, bias=b["bias"], out=ys)
                 else:
-                    _hxq.gemv(xs, idx, self._kcb, b["group_scale"], b["group_offset"],
-                              self.group_size, rp, col, delta, b["bias"], out=ys)
+                    _hxq.gemv(xs, idx, self._kernel_codebook(codebook), b["group_scale"],
+                              b["group_offset"], self.group_size, rp, col, delta, b["bias"], out=ys)
         if svd_on:
             xf = x2.float()
             out += ((xf @ b["svd_Vt"].t()) * b["svd_s"].unsqueeze(0)) @ b["svd_U"].t()

@@ -349,3 +349,36 @@ def test_tensors_assigned_as_parameters(dev, rows):
         # one fp32 rounding of the sum with the bias on either side: 2 ulp of |y| + 2
         bound = 2 * 2.0 ** -23 * (float(y.abs().max()) + 2)
         assert float((m(x) - (y + 1)).abs().max()) <= bound
+
+
+def _move_without_stub(m):
+    del m.weight                      # the stub that is a Parameter always
+    m.bias = torch.nn.Parameter(m.bias.clone(), requires_grad=False)
+
+
+def _move_parametrize(m):
+    torch.nn.utils.parametrize.register_parametrization(m, "codebook", torch.nn.Identity())
+
+
+def _move_plain(m):
+    t = m.group_scale
+    del m.group_scale
+    m.group_scale = t.clone()         # in the module's __dict__ now
+
+
+@pytest.mark.parametrize("rows", [1, 16])
+@pytest.mark.parametrize("move,name", [(_move_without_stub, "bias"), (_move_parametrize, "codebook"),
+                                       (_move_plain, "group_scale")])
+def test_tensors_kept_elsewhere_than_in_the_buffers(dev, move, name, rows):
+    T = synth.to_torch(synth.make_layer_np(96, 256, seed=4))
+    m = HelixLinear(256, 96, T["codebook"], T["indices"], T["sidecar_positions"],
+                    T["sidecar_values"], bias=torch.linspace(-0.5, 0.5, 96),
+                    group_scale=T["group_scale"], group_offset=T["group_offset"],
+                    group_size=T["group_size"]).to(dev)
+    x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(rows)).to(dev)
+    print(f"moved {name} rows={rows}", flush=True)
+    with torch.no_grad():
+        y = m(x)
+        move(m)
+        assert name not in m._buffers
+        assert torch.equal(m(x), y)
