@@ -1380,7 +1380,7 @@ extern "C" int hxq_select_f32(const float *x, int64_t n, const int64_t *ranks, i
 }
 
 extern "C" int64_t hxq_outliers_workspace_bytes(int64_t n) {
-    return 8 * std::max<int64_t>((n + kChunk - 1) / kChunk, 1) + 64;
+    return 8 * std::max<int64_t>((n + kChunk - 1) / kChunk, 1) + 64;  // 64: alignment
 }
 
 extern "C" int hxq_outliers_f32(const float *x, int64_t n, const float *lohi, int64_t capacity,
@@ -1394,9 +1394,9 @@ extern "C" int hxq_outliers_f32(const float *x, int64_t n, const float *lohi, in
     const int64_t chunks = (n + kChunk - 1) / kChunk;
     const dim3 grid(static_cast<uint32_t>((chunks + kWaves - 1) / kWaves));
     HXQ_REQUIRE((chunks + kWaves - 1) / kWaves < (int64_t{1} << 31), "n too large");
-    HXQ_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 7u) == 0, "workspace must be 8-byte aligned");
     const int vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
-    int64_t *cnt = static_cast<int64_t *>(workspace);
+    // (any alignment: the counts start at the next multiple of 8, in the spare bytes)
+    int64_t *cnt = reinterpret_cast<int64_t *>((reinterpret_cast<uintptr_t>(workspace) + 7u) & ~uintptr_t{7});
     hipLaunchKernelGGL(outlier_count_kernel, grid, dim3(kThreads), 0, stream, x, n, chunks, vec, lohi, cnt);
     HXQ_LAUNCH_CHECK();
     hipLaunchKernelGGL(outlier_scan_kernel, dim3(1), dim3(1024), 0, stream, cnt, chunks, count);

@@ -87,6 +87,26 @@ def test_select_and_outlier_edges(dev, n, offset):
         np.testing.assert_array_equal(val.cpu().numpy(), x[want])
 
 
+@pytest.mark.parametrize("shift", [0, 4, 1])
+def test_outliers_workspace_of_any_alignment(dev, shift):
+    n, lib = 9000, _hxq.lib()
+    x = torch.randn(n, generator=torch.Generator().manual_seed(2)).to(dev)
+    lohi = torch.tensor([-2.0, 2.0], device=dev)
+    size = int(lib.hxq_outliers_workspace_bytes(n))
+    buf = torch.full((size + 16,), 0x5a, dtype=torch.uint8, device=dev)
+    pos = torch.empty(n, dtype=torch.int64, device=dev)
+    val, cnt = torch.empty(n, device=dev), torch.empty(1, dtype=torch.int64, device=dev)
+    print(f"outliers workspace + {shift}", flush=True)
+    rc = lib.hxq_outliers_f32(x.data_ptr(), n, lohi.data_ptr(), n, pos.data_ptr(), val.data_ptr(),
+                              cnt.data_ptr(), buf.data_ptr() + shift, size,
+                              torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.hxq_last_error()
+    want = torch.nonzero(x.abs() > 2.0).ravel()
+    m = int(cnt)
+    assert torch.equal(pos[:m], want) and torch.equal(val[:m], x[want])
+    assert (buf[:shift] == 0x5a).all() and (buf[shift + size:] == 0x5a).all()
+
+
 @pytest.mark.parametrize("rows,cols,G", [(1, 16, 16), (3, 96, 96), (5, 260, 52), (7, 640, 128), (2, 384, 1)])
 def test_affine_fit_edges(dev, rows, cols, G):
     """Group counts that are no multiple of a wave's four, groups below, at and above a wave."""
