@@ -108,6 +108,15 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders the LDS accesses of one wave across its lanes: what any lane wrote
+// before is what any lane reads after.  LDS serves a wave in order, so this
+// costs no instruction; it keeps the compiler to that order.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Raw buffer resource over [base, base + bytes): loads at or past `bytes`
 // return zero (hardware range check).  bytes must fit in 32 bits.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, int64_t bytes) {

@@ -540,8 +540,7 @@ __global__ __launch_bounds__(kThreads) void km_sum_kernel(const float *sorted_va
                     const bool node = pairwise_path(m, at, off, len, depth);
                     if (node && depth > d) s_leaf[at] = s_leaf[at] + s_leaf[at + (1 << (kDepth - 1 - d))];
                 }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_order();
             }
         }
         __syncthreads();

@@ -454,18 +454,18 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
             // that entry is infinite and no weight uses it (the exit: at most 1 %, 16 x
             // 3584 x 18944 30.7 / 30.9 us, 64 x 3584 x 18944 52.2 / 52.1)
             if (SP > 1 && t + s >= nst) break;
-            // X through the wave's tile into operand layout (LDS serves a wave in order)
+            // X through the wave's tile into operand layout
             u32x4 xo[MT][XCH / 4];
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
 #pragma unroll
                 for (int q = 0; q < NX; ++q)
                     *reinterpret_cast<u32x4 *>(x_slot(lane / XCH + (64 / XCH) * q, lane % XCH)) = xv[s][i][q];
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_order();
 #pragma unroll
                 for (int q = 0; q < XCH / 4; ++q)
                     xo[i][q] = *reinterpret_cast<const u32x4 *>(x_slot(r16, (XCH / 4) * hq + q));
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_order();
             }
             load_x(tn + s, s);
             const uint32_t ao = a_base(tn + s);
