@@ -67,6 +67,16 @@ __device__ __forceinline__ uint16_t f32_to_f16(float f) {
     return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
 }
 
+// Two fp32 values rounded to nearest even to bf16 or fp16, in one conversion.
+template <bool BF16>
+__device__ __forceinline__ uint32_t pack16(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
+}
+
 // Native 4 x u32 vector (usable with the nontemporal load builtin).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -161,6 +171,46 @@ __device__ __forceinline__ float tbl_lookup0(uint32_t lane_off, uint32_t w) {
         addr = ((w >> (8 * B)) & 0xffu) * (NREP * 4) + lane_off;
     }
     return *reinterpret_cast<lds_cfloat *>(static_cast<uintptr_t>(addr));
+}
+
+// Inclusive scan of v over the wave by DPP (row_shr 1, 2, 4, 8 within rows,
+// then row_bcast:15 / :31 across them): no LDS round trips.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// Row tile rt (of bm rows, counted over all experts; expert e owns the sorted
+// rows [seg[e], seg[e + 1])) of a grouped launch: its expert, first row and the
+// segment's end; false past the last tile.  Every wave computes it alike (lanes
+// cover experts e, e + 64, ...; a scan of the experts' tile counts).
+__device__ __forceinline__ bool expert_row_tile(const int32_t *seg, int n_exp, int bm, int rt, int &e,
+                                                int &row0, int &rend) {
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int c0 = 0; c0 < n_exp; c0 += 64) {
+        const int ee = c0 + lane;
+        const int a = ee < n_exp ? seg[ee] : 0;
+        const int b = ee < n_exp ? seg[ee + 1] : 0;
+        const int nt = (b - a + bm - 1) / bm;
+        const int inc = wave_scan(nt);
+        const int tot = __builtin_amdgcn_readlane(inc, 63);
+        if (rt < base + tot) {
+            // wave-uniform results, in scalar registers (they form buffer bases)
+            const int l = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(base + inc > rt)));
+            e = c0 + l;
+            row0 = __builtin_amdgcn_readlane(a, l) + (rt - base - __builtin_amdgcn_readlane(inc - nt, l)) * bm;
+            rend = __builtin_amdgcn_readlane(b, l);
+            return true;
+        }
+        base += tot;
+    }
+    return false;
 }
 
 // Wave64 sum via DPP; the total lands in lane 63.

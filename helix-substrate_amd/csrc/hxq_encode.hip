@@ -244,17 +244,6 @@ __global__ __launch_bounds__(kThreads) void digit_count_kernel(DigitSrc src, int
     for (int j = threadIdx.x; j < kDigits; j += kThreads) blk[j * nblk + blockIdx.x] = cnt[j];
 }
 
-// Inclusive wave scan by DPP (row_shr 1, 2, 4, 8, then row_bcast 15 and 31).
-__device__ __forceinline__ int wave_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-    return v;
-}
-
 // blk[j][b] -> elements of bucket j in blocks before b; counts[j] = all of them
 __global__ __launch_bounds__(kThreads) void bucket_scan_kernel(int32_t *blk, int64_t nblk, int k, int32_t *counts,
                                                                const int32_t *done) {

@@ -41,11 +41,8 @@
 
 namespace hxq {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kConsumers = 4;                   // MFMA waves
@@ -104,14 +101,8 @@ __device__ __forceinline__ bool dense_tile(const GemmArgs &g, int b, int &tx, in
 }
 
 template <bool BF16>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
-}
-
-template <bool BF16>
 __device__ __forceinline__ uint16_t to16(float v) {
-    return static_cast<uint16_t>(pack2<BF16>(v, 0.f) & 0xffffu);
+    return static_cast<uint16_t>(pack16<BF16>(v, 0.f) & 0xffffu);
 }
 
 // Element offset of 16-byte chunk c (0..7) of LDS row r (64 elements, 128 B).
@@ -413,8 +404,8 @@ __global__ __launch_bounds__(kGemmThreads, 3) void gemm_kernel(const GemmArgs g)
                             const float c = lookup(part_of(i), w, b);
                             v[b] = AFFINE ? affine_fma(c, so[i].x, so[i].y) : c;
                         }
-                        pk[dd * 2] = pack2<BF16>(v[0], v[1]);
-                        pk[dd * 2 + 1] = pack2<BF16>(v[2], v[3]);
+                        pk[dd * 2] = pack16<BF16>(v[0], v[1]);
+                        pk[dd * 2 + 1] = pack16<BF16>(v[2], v[3]);
                     }
                     *reinterpret_cast<u32x4 *>(&sB[buf][swz(tile_row(i), qc * 2 + h)]) =
                         u32x4{pk[0], pk[1], pk[2], pk[3]};

@@ -67,16 +67,6 @@ __device__ __forceinline__ float silu(float v) {
     return v / d;
 }
 
-// Two fp32 values rounded to nearest even in one conversion.
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-template <bool BF16>
-__device__ __forceinline__ uint32_t pack16(float a, float b) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
-}
-
 // torch.nn.functional.softplus (beta 1, threshold 20)
 __device__ __forceinline__ float softplus(float v) { return v > 20.f ? v : log1pf(expf(v)); }
 

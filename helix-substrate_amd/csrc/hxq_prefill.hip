@@ -112,11 +112,8 @@ Plan plan(int64_t m, int64_t out, int64_t in, bool f32, bool affine, int32_t gro
 
 namespace pg {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
@@ -169,50 +166,8 @@ struct Args {
     const float *sc_val1;
 };
 
-// Row tile rt of a grouped launch: the expert e whose segment holds it, its
-// first sorted row and the segment end.  Every wave computes it alike (lanes
-// cover experts e, e + 64, ...; a wave scan of the per-expert tile counts).
-__device__ __forceinline__ bool grouped_tile(const Args &g, int bm, int rt, int &e, int &row0,
-                                             int &rend) {
-    const int lane = threadIdx.x & 63;
-    int base = 0;
-    for (int c0 = 0; c0 < g.n_exp; c0 += 64) {
-        const int ee = c0 + lane;
-        const int a = ee < g.n_exp ? g.seg[ee] : 0;
-        const int b = ee < g.n_exp ? g.seg[ee + 1] : 0;
-        const int nt = (b - a + bm - 1) / bm;
-        // inclusive scan of nt over the wave by DPP (row_shr 1, 2, 4, 8 within
-        // rows, then row_bcast:15 / :31 across them): no LDS round trips
-        int inc = nt;
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x111, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x112, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x114, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x118, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);
-        const int tot = __builtin_amdgcn_readlane(inc, 63);
-        if (rt < base + tot) {
-            const unsigned long long m = __ballot(base + inc > rt);
-            const int L = __builtin_amdgcn_readfirstlane(__builtin_ctzll(m));
-            // wave-uniform results, in scalar registers (they form buffer bases)
-            e = c0 + L;
-            row0 = __builtin_amdgcn_readlane(a, L) + (rt - base - __builtin_amdgcn_readlane(inc - nt, L)) * bm;
-            rend = __builtin_amdgcn_readlane(b, L);
-            return true;
-        }
-        base += tot;
-    }
-    return false;
-}
-
 template <bool BF16>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
-}
-
-template <bool BF16>
-__device__ __forceinline__ uint32_t to16(float v) { return pack2<BF16>(v, 0.f) & 0xffffu; }
+__device__ __forceinline__ uint32_t to16(float v) { return pack16<BF16>(v, 0.f) & 0xffffu; }
 
 // Element offset of 16-byte chunk c (0..7) of LDS row r (64 elements, 128 B).
 // gfx950's LDS has 64 banks and serves 16 lanes of a 16-byte access per
@@ -309,7 +264,7 @@ __global__ __launch_bounds__(kBN / (32 * NJ) * 64, BM == 64 ? 4 : 1) void prefil
         tx = j % g.grp_tiles_x;
         tl = rt * g.grp_tiles_x + tx;
         int e, row0, rend;
-        if (!grouped_tile(g, BM, rt, e, row0, rend)) return;  // block-uniform
+        if (!expert_row_tile(g.seg, g.n_exp, BM, rt, e, row0, rend)) return;  // block-uniform
         r0 = row0;
         mlim = rend;
         const bool b1 = tx * kBN >= g.out_split;
@@ -522,7 +477,7 @@ __global__ __launch_bounds__(kBN / (32 * NJ) * 64, BM == 64 ? 4 : 1) void prefil
                         v0 = affine_fma(v0, sc, of);
                         v1 = affine_fma(v1, sc, of);
                     }
-                    b[16 * j + 4 * s + t] = pack2<BF16>(v0, v1);
+                    b[16 * j + 4 * s + t] = pack16<BF16>(v0, v1);
                 }
                 continue;
             } else if constexpr (FMT == HXQ_FMT_VQ2_U16) {
@@ -532,7 +487,7 @@ __global__ __launch_bounds__(kBN / (32 * NJ) * 64, BM == 64 ? 4 : 1) void prefil
                 for (int t = 0; t < 4; ++t) {
                     const uint32_t w = qv[buf][NQ * j + (s >> 1)][2 * (s & 1) + (t >> 1)];
                     const float2 c = t2[(w >> (16 * (t & 1))) & (kPairCodes - 1u)];
-                    b[16 * j + 4 * s + t] = pack2<BF16>(c.x, c.y);
+                    b[16 * j + 4 * s + t] = pack16<BF16>(c.x, c.y);
                 }
                 continue;
             } else if constexpr (FMT == HXQ_FMT_VQ2_P12) {
@@ -541,7 +496,7 @@ __global__ __launch_bounds__(kBN / (32 * NJ) * 64, BM == 64 ? 4 : 1) void prefil
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float2 c = t2[field24(qv[buf][NQ * j], qv[buf][NQ * j + 1], 48 * s + 12 * t, 12)];
-                    b[16 * j + 4 * s + t] = pack2<BF16>(c.x, c.y);
+                    b[16 * j + 4 * s + t] = pack16<BF16>(c.x, c.y);
                 }
                 continue;
             } else if constexpr (FMT == HXQ_FMT_AF6) {
@@ -550,7 +505,7 @@ __global__ __launch_bounds__(kBN / (32 * NJ) * 64, BM == 64 ? 4 : 1) void prefil
                 for (int t = 0; t < 4; ++t) {
                     const float v0 = static_cast<float>(field24(qv[buf][NQ * j], qv[buf][NQ * j + 1], 48 * s + 12 * t, 6));
                     const float v1 = static_cast<float>(field24(qv[buf][NQ * j], qv[buf][NQ * j + 1], 48 * s + 12 * t + 6, 6));
-                    b[16 * j + 4 * s + t] = pack2<BF16>(affine_fma(v0, sc, of), affine_fma(v1, sc, of));
+                    b[16 * j + 4 * s + t] = pack16<BF16>(affine_fma(v0, sc, of), affine_fma(v1, sc, of));
                 }
                 continue;
             }
@@ -568,8 +523,8 @@ __global__ __launch_bounds__(kBN / (32 * NJ) * 64, BM == 64 ? 4 : 1) void prefil
                     v2 = affine_fma(v2, sc, of);
                     v3 = affine_fma(v3, sc, of);
                 }
-                b[16 * j + 2 * d] = pack2<BF16>(v0, v1);
-                b[16 * j + 2 * d + 1] = pack2<BF16>(v2, v3);
+                b[16 * j + 2 * d] = pack16<BF16>(v0, v1);
+                b[16 * j + 2 * d + 1] = pack16<BF16>(v2, v3);
             }
         }
     };

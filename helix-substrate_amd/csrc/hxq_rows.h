@@ -30,11 +30,8 @@
 namespace hxq {
 namespace rw {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
@@ -91,37 +88,6 @@ struct Grouped {
     int64_t idx_es, ga_es, scp_es;          // per-expert strides (codebooks: 256)
 };
 
-// Row tile rt (of bm rows, counted over all experts): its expert, first position
-// and the segment's end; false past the last one.  Every wave alike, by wave
-// scans.
-__device__ __forceinline__ bool row_tile(const Grouped &g, int bm, int rt, int &e, int &row0, int &rend) {
-    const int lane = threadIdx.x & 63;
-    int base = 0;
-    for (int c0 = 0; c0 < g.n_exp; c0 += 64) {
-        const int ee = c0 + lane;
-        const int a = ee < g.n_exp ? g.seg[ee] : 0;
-        const int b = ee < g.n_exp ? g.seg[ee + 1] : 0;
-        const int nt = (b - a + bm - 1) / bm;
-        int inc = nt;
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x111, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x112, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x114, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x118, 0xf, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
-        inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);
-        const int tot = __builtin_amdgcn_readlane(inc, 63);
-        if (rt < base + tot) {
-            const int l = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(base + inc > rt)));
-            e = c0 + l;
-            row0 = __builtin_amdgcn_readlane(a, l) + (rt - base - __builtin_amdgcn_readlane(inc - nt, l)) * bm;
-            rend = __builtin_amdgcn_readlane(b, l);
-            return true;
-        }
-        base += tot;
-    }
-    return false;
-}
-
 // index bytes per 16 weights
 __host__ __device__ constexpr int fmt_b16(int f) {
     return f == HXQ_FMT_SCALAR_U16 ? 32 : (f == HXQ_FMT_VQ2_P12 || f == HXQ_FMT_AF6) ? 12 : 16;
@@ -130,12 +96,6 @@ __host__ __device__ constexpr int fmt_table_bytes(int f) {
     return f == HXQ_FMT_SCALAR ? 256 * kNrep * 4
          : f == HXQ_FMT_SCALAR_U16 ? kPairCodes * 4
          : f == HXQ_FMT_AF6 ? 16 : kPairCodes * 8;
-}
-
-template <int XT>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    if constexpr (XT == 1) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
 }
 
 // MT: 16-row tiles of X; NS: subtiles per block (the grid's last block may own
@@ -181,7 +141,8 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
     int nnz = 0;
     if constexpr (GRP) {
         int e, w = blockIdx.x % (grp.runs * grp.n_banks);
-        if (!row_tile(grp, MT * kSub, blockIdx.x / (grp.runs * grp.n_banks), e, m0, mend)) return;  // block-uniform
+        if (!expert_row_tile(grp.seg, grp.n_exp, MT * kSub, blockIdx.x / (grp.runs * grp.n_banks), e, m0, mend))
+            return;  // block-uniform
         const Bank &b = grp.bank[w >= grp.runs];
         if (w >= grp.runs) {
             w -= grp.runs;
@@ -391,8 +352,8 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
         } else {
 #pragma unroll
             for (int d = 0; d < 8; ++d) {
-                if constexpr (AFF) b[d] = pack2<XT>(affine_fma(v[2 * d], sc, of), affine_fma(v[2 * d + 1], sc, of));
-                else b[d] = pack2<XT>(v[2 * d], v[2 * d + 1]);
+                if constexpr (AFF) b[d] = pack16<XT == 1>(affine_fma(v[2 * d], sc, of), affine_fma(v[2 * d + 1], sc, of));
+                else b[d] = pack16<XT == 1>(v[2 * d], v[2 * d + 1]);
             }
         }
     };
@@ -425,7 +386,7 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
             val = __float_as_uint(v);
         } else {
             code = owner | ((c & 15u) >> 1) << 8 | (c & 1u) << 16;
-            val = pack2<XT>(v, 0.f) & 0xffffu;
+            val = pack16<XT == 1>(v, 0.f) & 0xffffu;
         }
     };
     // chunk c of row m of the wave's X tile: the same bank swizzle as the
@@ -541,8 +502,8 @@ __global__ __launch_bounds__(W * 64, GRP ? 4 : 1) void rows_kernel(const uint8_t
         } else {
             uint16_t *y = static_cast<uint16_t *>(g.y) + o;
             uint32_t p0, p1;
-            if (g.y_dtype == HXQ_BF16) { p0 = pack2<1>(v[0], v[1]); p1 = pack2<1>(v[2], v[3]); }
-            else { p0 = pack2<0>(v[0], v[1]); p1 = pack2<0>(v[2], v[3]); }
+            if (g.y_dtype == HXQ_BF16) { p0 = pack16<true>(v[0], v[1]); p1 = pack16<true>(v[2], v[3]); }
+            else { p0 = pack16<false>(v[0], v[1]); p1 = pack16<false>(v[2], v[3]); }
             if (g.vec_out && nv == 4) {
                 *reinterpret_cast<uint2 *>(y) = make_uint2(p0, p1);
             } else {
