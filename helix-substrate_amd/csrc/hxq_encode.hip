@@ -941,13 +941,6 @@ static int grid_for(int64_t n) {
     return static_cast<int>(std::min<int64_t>(std::max<int64_t>(g, 1), 8192));
 }
 
-static int64_t next_pow2(int64_t n) {
-    int64_t p = 2048;
-    while (p < n) p <<= 1;
-    return p;
-}
-
-
 // ---------------------------------------------------------------------------
 // pair (vector_dim 2) codebook: nearest centroid and centroid update
 // ---------------------------------------------------------------------------
@@ -1212,7 +1205,10 @@ extern "C" int hxq_assign_nearest_wide(const float *x, int64_t n, const float *c
 }
 
 extern "C" int64_t hxq_sort_workspace_bytes(int64_t n) {
-    return n <= 0 ? 0 : 4 * next_pow2(n);
+    if (n <= 0) return 0;
+    int64_t p = 2048;
+    while (p < n) p <<= 1;
+    return 4 * p;
 }
 
 // Four 8-bit passes between keys and tmp (n keys each), ending in keys.

@@ -551,6 +551,8 @@ int hxq_argmax(const float *logits, int64_t n, int32_t *out_id, int32_t *pos,
  *   most `capacity` written.
  *   With hxq_select_f32 these replace find_outliers_percentile
  *   (helix_substrate/generate_sidecars_v3.py:18-40).
+ * hxq_sort_workspace_bytes: of no entry point any more (the sort's buffers are
+ *   part of hxq_kmeans_workspace_bytes); kept for callers that link it.
  */
 int hxq_assign_nearest(const float *x, int64_t n, const float *codebook, int32_t k,
                        uint8_t *indices, hipStream_t stream);
