@@ -151,6 +151,52 @@ def test_conv_split_16bit_vector_path(dev, W, L, pdt):
     assert torch.equal(cs16, cs32)
 
 
+@pytest.mark.parametrize("b,L,W,pdt", [
+    # 8 sequences: 16 steps per block, ending in a round's 1st, 2nd, 3rd step or with it
+    (8, 173, 4, torch.bfloat16), (8, 170, 4, torch.float16), (8, 171, 3, torch.bfloat16),
+    (8, 176, 2, torch.float16), (8, 177, 1, torch.bfloat16), (8, 164, 4, torch.bfloat16),
+    # 2 sequences: 8 steps
+    (2, 173, 4, torch.bfloat16), (2, 175, 4, torch.float16), (2, 170, 3, torch.float16),
+    (2, 169, 2, torch.bfloat16), (2, 172, 1, torch.bfloat16),
+])
+def test_conv_split_vector_rounds(dev, b, L, W, pdt):
+    """The vector kernel with several rounds of time steps per block and three blocks of channels
+    (the last one part full), against the scalar kernel as in the test above."""
+    I, G, N, H, d_mlp = 4096, 1, 128, 24, 8
+    cd = I + 2 * G * N
+    blocks = 3 * b * ((L + 15) // 16)       # at 16 steps; 256 compute units
+    assert (blocks >= 256) == (b == 8) and 4 * blocks >= 256
+    g = torch.Generator().manual_seed(W * 10 + L)
+    proj = torch.randn(b, L, 2 * d_mlp + 2 * I + 2 * G * N + H, generator=g).to(pdt)
+    w = (torch.randn(cd, W, generator=g) * 0.5).to(dev)
+    cb = (torch.randn(cd, generator=g) * 0.1).to(dev)
+    dtb = torch.randn(H, generator=g).to(dev)
+    print(f"conv_split rounds b={b} L={L} W={W} {pdt}", flush=True)
+    cs16, cs32 = (torch.full((b, cd, W), float("nan"), device=dev) for _ in range(2))
+    args = (w, cb, dtb, 1e-3, float("inf"), d_mlp, I, G, N, H)
+    got = _hxq.mamba2_conv_split(proj.to(dev), *args, conv_state=cs16)
+    ref = _hxq.mamba2_conv_split(proj.float().to(dev), *args, out_dtype=torch.float32, conv_state=cs32)
+    for t, r in zip(got[:3], ref[:3]):
+        assert torch.equal(t, r.to(pdt))
+    assert torch.equal(got[3], ref[3]) and torch.equal(cs16, cs32)
+
+
+@pytest.mark.parametrize("kind", ["transposed", "unaligned", "double"])
+def test_mixer_final_state_of_any_layout(dev, kind):
+    """A final state that the scan cannot write in place (strides, alignment, type) is copied."""
+    m, _, _, _ = _mixer(d_model=128, heads=4, head_dim=32, state=16, seed=5, device=dev)
+    x = torch.randn(2, 70, 128, generator=torch.Generator().manual_seed(1)).to(dev).to(torch.bfloat16)
+    conv, ssm = m.new_state(2, dev)
+    y = m(x, (conv, ssm))
+    conv2 = torch.zeros_like(conv)
+    h = {"transposed": torch.zeros(2, 4, 16, 32, device=dev).transpose(2, 3),
+         "unaligned": torch.zeros(2 * 4 * 32 * 16 + 1, device=dev)[1:].view(2, 4, 32, 16),
+         "double": torch.zeros(2, 4, 32, 16, device=dev, dtype=torch.float64)}[kind]
+    print(f"final state {kind}", flush=True)
+    assert torch.equal(m(x, (conv2, h)), y)
+    assert torch.equal(h.float(), ssm) and torch.equal(conv2, conv) and bool(ssm.any())
+
+
 @pytest.mark.parametrize("width,ydt,odt", [(4096, torch.float32, torch.bfloat16),
                                            (2048, torch.bfloat16, torch.float32),
                                            (8192, torch.float32, torch.float32)])
