@@ -87,7 +87,7 @@ def _gemm32(mod, x):
     (64, 256, 512),
     (300, 640, 1536),     # ragged M and OUT tiles
     (512, 512, 3584),     # Qwen2.5-7B kv shape
-    (1024, 384, 2048),    # 256-row tiles
+    (1024, 384, 2048),    # several 64-row blocks of the few-row kernel
 ])
 def test_gemm_bf16_matches_oracle(dev, m, out_f, in_f):
     L, T = _layer(out_f, in_f, seed=m + out_f, sigma=0.015)
@@ -134,11 +134,13 @@ def test_gemm_dense_sidecar_rows(dev):
     _check(_gemm32(mod, x.to(dev)), x, _oracle_w(L))
 
 
-def test_prefill_sidecar_dense_block_and_repeats(dev):
+@pytest.mark.parametrize("m,out_f,tiled", [(96, 256, False), (1001, 1000, True)])
+def test_prefill_sidecar_dense_block_and_repeats(dev, m, out_f, tiled):
     """A 64 x 64 block fully in the sidecar (4096 entries in one row group and
     K step: the per-step list overflows its 64-entry load), positions repeated
-    with new values (the last copy wins), under a K split."""
-    out_f, in_f, m = 1000, 512, 1001   # the tiled kernel
+    with new values (the last copy wins), in the few-row kernel and in the
+    tiled one under a K split."""
+    in_f = 512
     L = synth.make_layer_np(out_f, in_f, seed=21, sidecar=False)
     rs = np.random.RandomState(3)
     blk = (np.arange(64, 128)[:, None] * in_f + np.arange(128, 192)[None, :]).ravel()
@@ -152,7 +154,9 @@ def test_prefill_sidecar_dense_block_and_repeats(dev):
     W = _oracle_w(L)
     assert np.array_equal(W.exact.ravel()[rep], val[-50:])   # the last copy is the oracle's value
     x = torch.randn(m, in_f, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16)
-    assert _hxq.lib().hxq_prefill_gemm_plan(m, out_f, in_f, 1, _hxq.FMT_SCALAR, 128) > 0   # K is split
+    plan = _hxq.lib().hxq_prefill_gemm_plan(m, out_f, in_f, _hxq.dtype_code(x.dtype),
+                                            _hxq.FMT_SCALAR, 128)
+    assert plan > 0 if tiled else plan == -1
     _check(_gemm32(mod, x.to(dev)), x, W)
     y = mod(x.to(dev))
     assert mod._last_dispatch_path == "hip_gemm"

@@ -66,6 +66,16 @@ def test_rows_formats(dev, fmt, m, out, inp, xdt):
     _check(dev, fmt, m, out, inp, 128 if inp % 128 == 0 else 64, xdt)
 
 
+@pytest.mark.parametrize("fmt", [_hxq.FMT_SCALAR, _hxq.FMT_SCALAR_U16] + FMTS)
+@pytest.mark.parametrize("out", [6400, 11200, 18944])   # runs of 2, 3 and 5 (uint16: 3) subtiles
+@pytest.mark.parametrize("m", [5, 20, 40, 64])          # 1 to 4 row tiles (fp32: 1 or 2)
+def test_rows_every_run_and_row_tile(dev, fmt, out, m):
+    for xdt in [torch.bfloat16, torch.float32] if m != 64 else [torch.float16]:
+        assert _hxq.lib().hxq_prefill_gemm_plan(m, out, 192, _hxq.dtype_code(xdt), fmt,
+                                                0 if fmt in FMTS[:2] else 64) == -1
+        _check(dev, fmt, m, out, 192, 64, xdt)
+
+
 @pytest.mark.parametrize("m,out,inp", [(9, 130, 512), (20, 8200, 256)])
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
 def test_rows_dense_sidecar(dev, m, out, inp, xdt):
@@ -91,14 +101,22 @@ def test_rows_infinite_unused_entry(dev, m, out, inp, xdt):
     assert torch.isfinite(ys[0]).all() and torch.equal(ys[0], ys[1])
 
 
-@pytest.mark.parametrize("counts", [(1,), (0, 1, 0, 16), (17, 0, 3, 33), (0, 0, 5), (2, 2, 2, 2, 2, 2, 2)])
-@pytest.mark.parametrize("out,inp", [(64, 64), (336, 576), (1024, 2048)])
+_MANY = tuple((0, 1, 0, 0, 2, 0, 18)[e % 7] if e % 5 == 0 else e % 2 for e in range(150))
+
+
+@pytest.mark.parametrize("counts,out,inp", [
+    (c, out, inp) for out, inp in ((64, 64), (336, 576), (1024, 2048))
+    for c in ((1,), (0, 1, 0, 16), (17, 0, 3, 33), (0, 0, 5), (2, 2, 2, 2, 2, 2, 2),
+              (0, 17, 0, 0, 33, 0, 0, 1))] + [(_MANY, 64, 64)])
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
 def test_rows_grouped(dev, counts, out, inp, xdt):
-    """Experts of few, no and just over 16 rows; runs of five subtiles that end inside a block."""
+    """Experts of few, no and just over 16 or 32 rows, more experts than lanes of a wave; runs of
+    five subtiles that end inside a block.  (17, 0, 3, 33) is past the line: 64-row tiles."""
     from helix_substrate import synth
     from helix_substrate.moe import bank_to, stack_bank
     E, n = len(counts), sum(counts)
+    tile = _hxq.lib().hxq_moe_grouped_tile(n, E, _hxq.dtype_code(xdt), out, 64)
+    assert tile == (64 if counts == (17, 0, 3, 33) else 16)
     Ls = [synth.make_layer_np(out, inp, seed=e, group_size=64, density=0.01) for e in range(E)]
     bank = bank_to(stack_bank([synth.to_torch(L) for L in Ls]), dev)
     bank["group_size"] = 64
@@ -117,6 +135,30 @@ def test_rows_grouped(dev, counts, out, inp, xdt):
         W16 = torch.from_numpy(W).to(xdt).float().numpy()
         ref = oracle.linear_np(x[rows[lo:hi].long()].float().numpy(), W16)
         assert _maxrel(y[lo:hi], ref) <= 2e-5, e   # operands equal: order of fp32 sums
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_rows_paired_banks(dev, dt):
+    """Gate and up of one launch against the two run by themselves: the same sums, so what is
+    left is how the product gate / (1 + exp(-gate)) * up rounds to 16 bits (at most one step
+    of 2^-8 on a few of 256 terms)."""
+    from helix_substrate import moe
+    from test_gpu_moe import _bank, _skewed_logits
+    T, E, k, H, I = 25, 12, 3, 320, 256
+    bg, bu, bd = (_bank(E, o, i, seed=s, dev=dev, group_size=64)[1]
+                  for o, i, s in ((I, H, 10), (I, H, 30), (H, I, 50)))
+    for n_out in (I, H):
+        assert _hxq.lib().hxq_moe_grouped_tile(T * k, E, _hxq.dtype_code(dt), n_out, 64) == 16
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(3)).to(dt).to(dev)
+    r = _hxq.moe_route(_skewed_logits(T, E, 2, dev), k, False)
+    print(f"paired banks {dt}", flush=True)
+    y = _hxq.moe_ffn(x, r, bg, bu, bd, out_dtype=torch.float32)
+    gate, up = (_hxq.moe_grouped_gemm(x, r.sorted_rows, r.expert_offsets, b, T * k, out_dtype=dt).float()
+                for b in (bg, bu))
+    act = (torch.nn.functional.silu(gate) * up).to(dt)
+    o = _hxq.moe_grouped_gemm(act, None, r.expert_offsets, bd, T * k, out_dtype=dt).float()
+    ref = (o[r.assign_pos.long().view(T, k)] * r.topk_weights.view(T, k, 1)).sum(1)
+    assert float((y - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
 
 
 def test_rows_allocate_nothing(dev):
