@@ -9,6 +9,7 @@ torch's current HIP stream of the tensor's device.  A non-zero status raises
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from pathlib import Path
 
@@ -493,11 +494,19 @@ def prefill_gemm(x, indices, codebook, group_affine, group_size, sc_grp_ptr, sc_
     return out
 
 
+@functools.lru_cache(maxsize=1024)
+def _prefill_plan(m, out_f, in_f, xdt, fmt, group, device):
+    """hxq_prefill_gemm_plan on `device`, the current one (the plan counts its compute units): a
+    function of these numbers, asked once for each (1 us a call otherwise).  -1: the few-row
+    kernel, which takes no workspace."""
+    return lib().hxq_prefill_gemm_plan(m, out_f, in_f, xdt, fmt, group)
+
+
 def _prefill_call(L, x, m, out_f, in_f, fmt, indices, codebook, n_codes, group_affine, group_size,
                   sc_grp_ptr, sc_grp_key, sc_grp_val, bias, out):
     xdt = dtype_code(x.dtype)
-    # -1: the few-row kernel, which takes no workspace
-    nbytes = L.hxq_prefill_gemm_plan(m, out_f, in_f, xdt, fmt, 0 if group_affine is None else int(group_size))
+    nbytes = _prefill_plan(m, out_f, in_f, xdt, fmt, 0 if group_affine is None else int(group_size),
+                           x.get_device())
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes > 0 else None
     return L.hxq_prefill_gemm(_ptr(x), xdt, fmt, _ptr(indices), _ptr(codebook),
                               n_codes, _ptr(group_affine), int(group_size), _ptr(sc_grp_ptr),
