@@ -681,9 +681,16 @@ def moe_ffn(x, routing, gate, up, down, out_dtype=None):
 # ---------------------------------------------------------------------------
 # Mamba2 mixer pieces
 # ---------------------------------------------------------------------------
+def _need_heads(d_inner, heads):
+    # the kernels write rows of d_inner channels into [heads, d_inner // heads]
+    if heads < 1 or d_inner % heads:
+        raise ValueError(f"d_inner ({d_inner}) must be a multiple of heads ({heads})")
+
+
 def mamba2_conv_split(proj, conv_w, conv_b, dt_bias, dt_min, dt_max, d_mlp, d_inner, ngroups,
                       state, heads, out_dtype=None, conv_state=None):
     """proj [b, L, proj_width] -> x [b, L, heads, d_inner/heads], B, C [b, L, G, N], dt [b, L, H]."""
+    _need_heads(d_inner, heads)
     b, L, pw = proj.shape
     width = conv_w.shape[1]
     od = out_dtype or proj.dtype
@@ -705,6 +712,7 @@ def mamba2_conv_split(proj, conv_w, conv_b, dt_bias, dt_min, dt_max, d_mlp, d_in
 def mamba2_conv_step(proj, conv_state, conv_w, conv_b, dt_bias, dt_min, dt_max, d_mlp, d_inner,
                      ngroups, state, heads, out_dtype=None):
     """One token: proj [b, proj_width]; conv_state fp32 [b, conv_dim, width] updated in place."""
+    _need_heads(d_inner, heads)
     b, pw = proj.shape
     width = conv_w.shape[1]
     od = out_dtype or proj.dtype

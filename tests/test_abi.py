@@ -88,3 +88,18 @@ def test_scan_workspace_query(lib):
     n = lib.hxq_ssm_scan_workspace_bytes(8, 2048, 64, 64, 128, 256)
     assert n >= 8 * 8 * 64 * 64 * 128 * 4
     assert lib.hxq_ssm_scan_workspace_bytes(0, 1, 1, 1, 1, 1) == -1
+
+
+def test_conv_refuses_heads_that_do_not_divide_the_channels():
+    """x is [heads, d_inner // heads] per token: too small a buffer for the kernel otherwise."""
+    import torch
+
+    from helix_substrate import _hxq
+
+    w = torch.zeros(96, 4)
+    for heads in (24, 0):
+        args = (w, None, None, 0.0, float("inf"), 0, 64, 1, 16, heads)
+        with pytest.raises(ValueError, match="multiple of heads"):
+            _hxq.mamba2_conv_split(torch.zeros(1, 2, 2 * 64 + 32 + 24), *args)
+        with pytest.raises(ValueError, match="multiple of heads"):
+            _hxq.mamba2_conv_step(torch.zeros(1, 2 * 64 + 32 + 24), torch.zeros(1, 96, 4), *args)
