@@ -541,7 +541,7 @@ extern "C" int hxq_mamba2_conv_split(const void *proj, int32_t proj_dtype, const
     a.width = (int32_t)width; a.proj_dt = proj_dtype; a.out_dt = out_dtype;
     const int channels = a.d_inner + 2 * a.gn + a.heads;
     // 16-bit proj and outputs, channel counts / offsets multiples of 8, 16-byte
-    // aligned buffers, W <= 4: the 8-channel vector kernel plus the dt kernel
+    // aligned buffers, W <= 4: the 8-channel vector kernel, dt channels too
     const bool vec = proj_dtype != HXQ_F32 && out_dtype == proj_dtype && width <= 4 &&
                      a.proj_width % 8 == 0 && a.xbc_off % 8 == 0 && a.d_inner % 8 == 0 &&
                      a.gn % 8 == 0 &&
@@ -553,13 +553,16 @@ extern "C" int hxq_mamba2_conv_split(const void *proj, int32_t proj_dtype, const
     if (vec) {
         const int groups = (a.d_inner + 2 * a.gn) / 8;
         // 16 steps per block (taps and window read once in 16) while that gives
-        // every CU a block, fewer below: us at 16 / 8 / 4 steps, 4352 channels:
-        // 8 x 2048 tokens 97 / 105 / 125, 2 x 1000 18.9 / 22.0 / 22.4, 512
-        // 14.4 / 11.5 / 11.7, 64 12.2 / 9.1 / 7.6
+        // every CU two blocks, 8 while it gives one, else 4: us at 16 / 8 / 4 steps,
+        // 4352 channels: 8 x 2048 tokens 107 / 113 / 128, 4 x 700 (528 blocks of 16)
+        // 26.9 / 27.4 / 28.5; 2 x 1000 (378) 22.8 / 20.8 / 23.0, 1400 (264) 22.1 /
+        // 17.1 / 18.4; 1000 (189) 16.8 / 13.4 / 13.2, 512 15.8 / 9.9 / 8.6, 64 15.3 /
+        // 8.9 / 6.1; within a mixer, whose projection is not in the caches, 2 x 1000
+        // 266 at 16 and at 8, 1400 241.5 / 238.7 / 240.3, 512 140.3 / 135.2 / 133.0
         const int gx = (groups + 255) / 256;
         const int64_t blocks = static_cast<int64_t>(gx) * a.batch * ((a.seqlen + kConvT - 1) / kConvT);
         const int cus = device_cu_count();
-        a.steps = blocks >= cus ? kConvT : 4 * blocks >= cus ? kConvT / 2 : kConvTB;
+        a.steps = blocks >= 2 * cus ? kConvT : blocks >= cus ? kConvT / 2 : kConvTB;
         const dim3 grid(gx + 1, (a.seqlen + a.steps - 1) / a.steps, a.batch);
         const bool bf = proj_dtype == HXQ_BF16;
         switch (width) {

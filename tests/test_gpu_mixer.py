@@ -152,20 +152,21 @@ def test_conv_split_16bit_vector_path(dev, W, L, pdt):
 
 
 @pytest.mark.parametrize("b,L,W,pdt", [
-    # 8 sequences: 16 steps per block, ending in a round's 1st, 2nd, 3rd step or with it
-    (8, 173, 4, torch.bfloat16), (8, 170, 4, torch.float16), (8, 171, 3, torch.bfloat16),
-    (8, 176, 2, torch.float16), (8, 177, 1, torch.bfloat16), (8, 164, 4, torch.bfloat16),
-    # 2 sequences: 8 steps
-    (2, 173, 4, torch.bfloat16), (2, 175, 4, torch.float16), (2, 170, 3, torch.float16),
-    (2, 169, 2, torch.bfloat16), (2, 172, 1, torch.bfloat16),
+    # 16 sequences: 16 steps per block, ending in a round's 1st, 2nd, 3rd step or with it
+    (16, 173, 4, torch.bfloat16), (16, 170, 4, torch.float16), (16, 171, 3, torch.bfloat16),
+    (16, 176, 2, torch.float16), (16, 177, 1, torch.bfloat16), (16, 164, 4, torch.bfloat16),
+    # 8 sequences: 8 steps
+    (8, 173, 4, torch.bfloat16), (8, 175, 4, torch.float16), (8, 170, 3, torch.float16),
+    (8, 169, 2, torch.bfloat16), (8, 172, 1, torch.bfloat16),
+    (2, 173, 4, torch.bfloat16),   # 4 steps: one round
 ])
 def test_conv_split_vector_rounds(dev, b, L, W, pdt):
     """The vector kernel with several rounds of time steps per block and three blocks of channels
     (the last one part full), against the scalar kernel as in the test above."""
-    I, G, N, H, d_mlp = 4096, 1, 128, 24, 8
+    I, G, N, H, d_mlp = 4096, 1, 128, 32, 8
     cd = I + 2 * G * N
     blocks = 3 * b * ((L + 15) // 16)       # at 16 steps; 256 compute units
-    assert (blocks >= 256) == (b == 8) and 4 * blocks >= 256
+    assert blocks // 256 == {16: 2, 8: 1, 2: 0}[b]
     g = torch.Generator().manual_seed(W * 10 + L)
     proj = torch.randn(b, L, 2 * d_mlp + 2 * I + 2 * G * N + H, generator=g).to(pdt)
     w = (torch.randn(cd, W, generator=g) * 0.5).to(dev)
